@@ -259,6 +259,9 @@ _SIGS = {
     "fsg_cnn_conv3x3": (C.c_int, [P(fsg_cnn_conv), vp]),
     "fsg_cnn_conv3x3_wgrad": (C.c_int, [vp, vp, C.c_int32, C.c_int32, C.c_int32, C.c_int32, vp,
                                         vp, vp]),
+    "fsg_cnn_wgrad_workspace_size": (C.c_size_t, [C.c_int32, C.c_int32, C.c_int32]),
+    "fsg_cnn_conv3x3_wgrad_ws": (C.c_int, [vp, vp, C.c_int32, C.c_int32, C.c_int32, C.c_int32, vp,
+                                           vp, vp, C.c_size_t, vp]),
     "fsg_cnn_pack": (C.c_int, [vp, C.c_int32, C.c_int32, vp, C.c_int32, vp, C.c_int32, vp]),
     "fsg_cnn_adam": (C.c_int, [vp, vp, vp, vp, C.c_int32, C.c_float, C.c_float, C.c_float,
                                C.c_float, C.c_int32, vp]),

@@ -147,84 +147,209 @@ __global__ void __launch_bounds__(256) k_conv3x3(ConvArgs A) {
 
 // dW[co][ci][tap] += sum_p dz[p][co] * x[p + off(tap)][ci], db[co] += sum_p dz[p][co]
 // (the master-weight layout, w[co][ci][3][3]).
-// MFMA with M = output channel, N = input channel, K = 16 pixels per step.
-// A workgroup stages one 64-pixel row segment of dz and the three x rows
-// around it (zero outside the image) in LDS; wave w owns taps w, w+4, w+8.
+// MFMA with M = output channel, N = input channel, K = 16 pixels per step, so
+// both operands are wanted pixel-minor: they are transposed on their way into
+// LDS (a thread takes 8 pixels of a channel pair and writes each channel's 8
+// as one 16-byte word).  A workgroup takes WG_ROWS = 4 dz rows of a column
+// strip at a time, with the WG_ROWS + 2 x rows around them; wave r owns dz row
+// r and all nine taps.  Summing over the x pixel q = p + dx - 1 leaves x
+// unshifted and shifts dz instead: the two shifted operands come from the
+// aligned one and its neighbouring dwords by alignbit, so a k-step is two
+// 16-byte and two 4-byte LDS reads of dz and three of x for 9 + 1 MFMAs (the
+// tenth, against ones, sums dz for db).
+// Bound: loads in flight while staging (one or two blocks per CU); the MFMAs
+// of 32 80 x 80 patches take under 5 us.  A block's sums meet in LDS and leave
+// as one partial, which k_wgrad_reduce adds up: float atomics of every block's
+// 9216 sums to the same addresses were the bound before (1024 blocks: 469 us a
+// layer at 32 x 80 x 80 cells; now 21 and 8).
 struct WgradArgs {
   const u16* x;   // [B][H][W][cin]
   const u16* dz;  // [B][H][W][32]
-  float* dw;      // [cout][cin][9] f32 (accumulated), cout = 32
-  float* db;      // [32] f32 (accumulated)
+  float* part;    // [blocks][WG_PART]: sums by (tap, accumulator entry, lane), or
+  float* dw;      // (part NULL) every block adds to dw and db itself
+  float* db;
   int B, H, W, cin;
+  int sw, n_strips, n_rg;   // strip width (a multiple of 16), strips, row groups
 };
 
-constexpr int WG_SEG = 64;
+constexpr int WG_ROWS = 4;
+constexpr int WG_SW = 96;                 // widest strip
+constexpr int WG_XP = WG_SW + 8;          // pitch of a channel's pixels: 52 and 56 dwords,
+constexpr int WG_ZP = WG_SW + 16;         // whose multiples spread 16-byte reads over the banks
+constexpr int WG_XROW = CNN_C * WG_XP;    // u16 of one staged x row
+constexpr int WG_ZROW = CNN_C * WG_ZP;    // dz pixel q at q + 8 (one halo pixel each side)
+constexpr int WG_LDS = ((WG_ROWS + 2) * WG_XROW + WG_ROWS * WG_ZROW) * 2;
+constexpr int WG_PART = 10 * 1024;        // nine taps and the bias sums, 32 x 32 each
 
-__global__ void __launch_bounds__(256) k_conv3x3_wgrad(WgradArgs A) {
-  __shared__ __attribute__((aligned(16))) u16 sdz[WG_SEG * CNN_C];          // [px][co]
-  __shared__ __attribute__((aligned(16))) u16 sx[3 * (WG_SEG + 2) * CNN_C]; // [r][px][ci]
-  const int t = threadIdx.x;
-  const int lane = t & 63, wave = t >> 6;
-  const int n = lane & 31, half = lane >> 5;  // n: A row = co, B column = ci
-  const int segs_x = (A.W + WG_SEG - 1) / WG_SEG;
-  const int n_segs = A.B * A.H * segs_x;
-  f32x16 acc[3] = {{}, {}, {}};
-  float bsum = 0.0f;
-  for (int sg = blockIdx.x; sg < n_segs; sg += gridDim.x) {
-    const int sx0 = (sg % segs_x) * WG_SEG;
-    const int row = sg / segs_x;
-    const int b = row / A.H, y = row - b * A.H;
-    __syncthreads();
-    for (int e = t; e < WG_SEG * CNN_C; e += 256) {
-      const int p = e / CNN_C, c = e - p * CNN_C;
-      const int xx = sx0 + p;
-      sdz[e] = (xx < A.W) ? A.dz[(((int64_t)b * A.H + y) * A.W + xx) * CNN_C + c] : (u16)0;
-    }
-    for (int e = t; e < 3 * (WG_SEG + 2) * A.cin; e += 256) {
-      const int r = e / ((WG_SEG + 2) * A.cin);
-      const int rem = e - r * (WG_SEG + 2) * A.cin;
-      const int p = rem / A.cin, c = rem - p * A.cin;
-      const int yy = y + r - 1, xx = sx0 + p - 1;
-      sx[(r * (WG_SEG + 2) + p) * CNN_C + c] =
-          (yy >= 0 && yy < A.H && xx >= 0 && xx < A.W)
-              ? A.x[(((int64_t)b * A.H + yy) * A.W + xx) * A.cin + c]
-              : (u16)0;
-    }
-    __syncthreads();
-    if (t < CNN_C)
-      for (int p = 0; p < WG_SEG; p++) bsum += bf2f(sdz[p * CNN_C + t]);
+__device__ __forceinline__ bf16x8 bf8(unsigned a, unsigned b, unsigned c, unsigned d) {
+  return __builtin_bit_cast(bf16x8, make_uint4(a, b, c, d));
+}
+
+// two channels of a pixel; the tensors need no more than their own alignment
+__device__ __forceinline__ unsigned wg_pair(const u16* p) {
+  unsigned v;
+  __builtin_memcpy(&v, p, sizeof(v));
+  return v;
+}
+
+// 8 pixels x 2 channels (one dword per pixel) -> each channel's 8 as 16 bytes
+__device__ __forceinline__ void wg_transpose(const unsigned (&v)[8], uint4& lo, uint4& hi) {
+  lo = make_uint4(__builtin_amdgcn_perm(v[1], v[0], 0x05040100u),
+                  __builtin_amdgcn_perm(v[3], v[2], 0x05040100u),
+                  __builtin_amdgcn_perm(v[5], v[4], 0x05040100u),
+                  __builtin_amdgcn_perm(v[7], v[6], 0x05040100u));
+  hi = make_uint4(__builtin_amdgcn_perm(v[1], v[0], 0x07060302u),
+                  __builtin_amdgcn_perm(v[3], v[2], 0x07060302u),
+                  __builtin_amdgcn_perm(v[5], v[4], 0x07060302u),
+                  __builtin_amdgcn_perm(v[7], v[6], 0x07060302u));
+}
+
+// Entry o = (tap, accumulator entry e = 4i + j, lane l) of a partial, added to
+// its place: column ci = l % 32, row co = 8i + (l / 32) * 4 + j; tap 9 is db.
+__device__ __forceinline__ void wg_add(int o, int cin, float v, float* __restrict__ dw,
+                                       float* __restrict__ db) {
+  const int tap = o >> 10, e = (o >> 6) & 15, l = o & 63;
+  const int ci = l & 31, co = 8 * (e >> 2) + (l >> 5) * 4 + (e & 3);
+  if (tap < 9) {
+    if (ci < cin) atomicAdd(&dw[(co * cin + ci) * 9 + tap], v);
+  } else if (ci == 0) {
+    atomicAdd(&db[co], v);
+  }
+}
+
+__global__ void __launch_bounds__(256, 2) k_conv3x3_wgrad(WgradArgs A) {
+  extern __shared__ __attribute__((aligned(16))) u16 wl[];
+  u16* const sx = wl;                               // [row][ci][q]
+  u16* const sz = wl + (WG_ROWS + 2) * WG_XROW;     // [row][co][q + 8]
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int n = lane & 31, half = lane >> 5;        // n: A row = co, B column = ci
+  const int cp = A.cin >> 1;                        // channel pairs of x: 4 or 16
+  const int cps = cp == 16 ? 4 : 2;
+  const int ng = A.sw >> 3, n_ks = A.sw >> 4;
+  const int n_tasks = A.B * A.n_rg * A.n_strips;
+  f32x16 acc[10];
 #pragma unroll
-    for (int q = 0; q < 3; q++) {
-      const int tap = wave + 4 * q;
-      if (tap >= 9) continue;
-      const int dy = tap / 3, dx = tap % 3;  // staged row dy, column offset dx
-      for (int ks = 0; ks < WG_SEG / 16; ks++) {
-        bf16x8 a, bb;
+  for (int k = 0; k < 10; k++) acc[k] = f32x16{};
+  const unsigned one2 = 0x3f803f80u;
+  const bf16x8 ones = bf8(one2, one2, one2, one2);
+  // channels past cin stay zero in every staged row
+  if (A.cin < CNN_C)
+    for (int e = t; e < (WG_ROWS + 2) * WG_XROW / 8; e += 256)
+      *(uint4*)(sx + e * 8) = make_uint4(0, 0, 0, 0);
+  for (int task = blockIdx.x; task < n_tasks; task += gridDim.x) {
+    const int strip = task % A.n_strips, rem = task / A.n_strips;
+    const int b = rem / A.n_rg, y0 = (rem - b * A.n_rg) * WG_ROWS;
+    const int q0 = strip * A.sw;
+    __syncthreads();
+    // x rows y0 - 1 .. y0 + WG_ROWS, zero outside the image
+    for (int e = t; e < (WG_ROWS + 2) * ng << cps; e += 256) {
+      const int c2 = e & (cp - 1), rg = e >> cps;
+      const int r = rg / ng, g = rg - r * ng;
+      const int yy = y0 + r - 1, q = q0 + g * 8;
+      unsigned v[8];
+      const bool row_ok = yy >= 0 && yy < A.H;
+      const u16* p = A.x + (((int64_t)b * A.H + yy) * A.W + q) * A.cin + 2 * c2;
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-          const int p = ks * 16 + half * 8 + e;
-          a[e] = __builtin_bit_cast(__bf16, sdz[p * CNN_C + n]);
-          bb[e] = (n < A.cin) ? __builtin_bit_cast(__bf16, sx[(dy * (WG_SEG + 2) + p + dx) * CNN_C + n])
-                              : __builtin_bit_cast(__bf16, (u16)0);
-        }
-        acc[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bb, acc[q], 0, 0, 0);
+      for (int k = 0; k < 8; k++)
+        v[k] = row_ok && q + k < A.W ? wg_pair(p + k * A.cin) : 0u;
+      uint4 lo, hi;
+      wg_transpose(v, lo, hi);
+      u16* d = sx + r * WG_XROW + 2 * c2 * WG_XP + g * 8;
+      *(uint4*)d = lo;
+      *(uint4*)(d + WG_XP) = hi;
+    }
+    // dz rows y0 .. y0 + WG_ROWS - 1
+    for (int e = t; e < WG_ROWS * ng * 16; e += 256) {
+      const int c2 = e & 15, rg = e >> 4;
+      const int r = rg / ng, g = rg - r * ng;
+      const int yy = y0 + r, q = q0 + g * 8;
+      unsigned v[8];
+      const u16* p = A.dz + (((int64_t)b * A.H + yy) * A.W + q) * CNN_C + 2 * c2;
+#pragma unroll
+      for (int k = 0; k < 8; k++)
+        v[k] = yy < A.H && q + k < A.W ? wg_pair(p + k * CNN_C) : 0u;
+      uint4 lo, hi;
+      wg_transpose(v, lo, hi);
+      u16* d = sz + r * WG_ZROW + 2 * c2 * WG_ZP + 8 + g * 8;
+      *(uint4*)d = lo;
+      *(uint4*)(d + WG_ZP) = hi;
+    }
+    // the dz halo: pixel q0 - 1 at index 7, pixel q0 + sw at index 8 + sw
+    for (int e = t; e < WG_ROWS * 2 * CNN_C; e += 256) {
+      const int c = e & 31, side = (e >> 5) & 1, r = e >> 6;
+      const int yy = y0 + r, q = side ? q0 + A.sw : q0 - 1;
+      const bool ok = yy < A.H && q >= 0 && q < A.W;
+      sz[r * WG_ZROW + c * WG_ZP + (side ? 8 + A.sw : 7)] =
+          ok ? A.dz[(((int64_t)b * A.H + yy) * A.W + q) * CNN_C + c] : (u16)0;
+    }
+    __syncthreads();
+    // dz row `wave` against staged x rows wave + dy
+    const u16* zr = sz + wave * WG_ZROW + n * WG_ZP + 8 + half * 8;
+    const u16* xr = sx + wave * WG_XROW + n * WG_XP + half * 8;
+    for (int ks = 0; ks < n_ks; ks++) {
+      const uint4 v = *(const uint4*)(zr + ks * 16);
+      const unsigned pv = *(const unsigned*)(zr + ks * 16 - 2);
+      const unsigned nx = *(const unsigned*)(zr + ks * 16 + 8);
+      bf16x8 z[3];   // dx = 0, 1, 2: dz[q + 1], dz[q], dz[q - 1]
+      z[0] = bf8(__builtin_amdgcn_alignbit(v.y, v.x, 16), __builtin_amdgcn_alignbit(v.z, v.y, 16),
+                 __builtin_amdgcn_alignbit(v.w, v.z, 16), __builtin_amdgcn_alignbit(nx, v.w, 16));
+      z[1] = __builtin_bit_cast(bf16x8, v);
+      z[2] = bf8(__builtin_amdgcn_alignbit(v.x, pv, 16), __builtin_amdgcn_alignbit(v.y, v.x, 16),
+                 __builtin_amdgcn_alignbit(v.z, v.y, 16), __builtin_amdgcn_alignbit(v.w, v.z, 16));
+#pragma unroll
+      for (int dy = 0; dy < 3; dy++) {
+        const bf16x8 xb = *(const bf16x8*)(xr + dy * WG_XROW + ks * 16);
+#pragma unroll
+        for (int dx = 0; dx < 3; dx++)
+          acc[dy * 3 + dx] =
+              __builtin_amdgcn_mfma_f32_32x32x16_bf16(z[dx], xb, acc[dy * 3 + dx], 0, 0, 0);
       }
+      acc[9] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(z[1], ones, acc[9], 0, 0, 0);
     }
   }
-  // accumulate: lane holds column ci = n, rows co = 8i + half*4 + j
+  // the four waves' sums, one accumulator at a time through LDS
+  float* const red = (float*)wl;   // [2][4][1024]
+  float* const part = A.part ? A.part + (int64_t)blockIdx.x * WG_PART : nullptr;
 #pragma unroll
-  for (int q = 0; q < 3; q++) {
-    const int tap = wave + 4 * q;
-    if (tap >= 9 || n >= A.cin) continue;
+  for (int k = 0; k < 10; k++) {
+    float* buf = red + (k & 1) * 4096;
+    if (k == 0) __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int e = 0; e < 16; e++) buf[wave * 1024 + e * 64 + lane] = acc[k][e];
+    __syncthreads();
 #pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const int co = 8 * i + half * 4 + j;
-        atomicAdd(&A.dw[(co * A.cin + n) * 9 + tap], acc[q][4 * i + j]);
-      }
+    for (int e = 0; e < 4; e++) {
+      const int o = e * 256 + t;
+      const float v = (buf[o] + buf[1024 + o]) + (buf[2048 + o] + buf[3072 + o]);
+      if (part)
+        part[k * 1024 + o] = v;
+      else
+        wg_add(k * 1024 + o, A.cin, v, A.dw, A.db);
+    }
   }
-  if (t < CNN_C) atomicAdd(&A.db[t], bsum);
+}
+
+// dw, db += the blocks' partials: 64 entries per workgroup, its four waves
+// taking every fourth block (coalesced 256-byte reads), a fixed order.
+__global__ void __launch_bounds__(256)
+k_wgrad_reduce(const float* __restrict__ part, int n_part, int cin, float* __restrict__ dw,
+               float* __restrict__ db) {
+  __shared__ float red[4][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int o = blockIdx.x * 64 + lane;
+  float s = 0.0f;
+  int k = wave;
+  for (; k + 28 < n_part; k += 32) {
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) v[u] = part[(int64_t)(k + 4 * u) * WG_PART + o];
+    s += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+  }
+  for (; k < n_part; k += 4) s += part[(int64_t)k * WG_PART + o];
+  red[wave][lane] = s;
+  __syncthreads();
+  if (wave) return;
+  wg_add(o, cin, (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]), dw, db);
 }
 
 // Pack float32 master weights w[co][ci][3][3] into the forward layout
@@ -924,20 +1049,72 @@ extern "C" int fsg_cnn_conv3x3(const fsg_cnn_conv* c, void* stream) {
   return FSG_OK;
 }
 
+// Strips of at most WG_SW columns, equal and a multiple of 16; max_blocks
+// blocks at most take the (strip, row group) tasks in equal shares, so that
+// none is left with one task more in a second round.
+static int wgrad_plan(int batch, int h, int w, int max_blocks, WgradArgs& A) {
+  A.B = batch;
+  A.H = h;
+  A.W = w;
+  A.n_strips = (w + WG_SW - 1) / WG_SW;
+  A.sw = ((w + A.n_strips - 1) / A.n_strips + 15) / 16 * 16;
+  A.n_strips = (w + A.sw - 1) / A.sw;
+  A.n_rg = (h + WG_ROWS - 1) / WG_ROWS;
+  const int64_t tasks = (int64_t)batch * A.n_rg * A.n_strips;
+  const int64_t per = (tasks + max_blocks - 1) / max_blocks;
+  return tasks > 0x7fffffff ? 0 : (int)((tasks + per - 1) / per);
+}
+// Two blocks a CU (their staging LDS) where each writes a partial; 128 where
+// each adds its 9248 sums to the same addresses atomically (about 20 G/s).
+constexpr int WG_BLOCKS = 512, WG_BLOCKS_ATOMIC = 128;
+
+static int wgrad_run(const void* x, const void* dz, int32_t batch, int32_t h, int32_t w,
+                     int32_t cin, float* dw, float* db, float* part, size_t part_bytes,
+                     void* stream) {
+  if (!x || !dz || !dw || !db)
+    return fail(FSG_E_INVALID, "fsg_cnn_conv3x3_wgrad: NULL argument");
+  if (batch <= 0 || h <= 0 || w <= 0 || (cin != 8 && cin != 32))
+    return fail(FSG_E_INVALID, "fsg_cnn_conv3x3_wgrad: bad shape");
+  WgradArgs A{};
+  A.x = (const u16*)x;
+  A.dz = (const u16*)dz;
+  A.part = part;
+  A.dw = dw;
+  A.db = db;
+  A.cin = cin;
+  const int grid = wgrad_plan(batch, h, w, part ? WG_BLOCKS : WG_BLOCKS_ATOMIC, A);
+  if (grid <= 0) return fail(FSG_E_INVALID, "fsg_cnn_conv3x3_wgrad: too many pixels");
+  if (part && part_bytes < (size_t)grid * WG_PART * sizeof(float))
+    return fail(FSG_E_WORKSPACE, "fsg_cnn_conv3x3_wgrad: workspace too small");
+  hipStream_t s = as_stream(stream);
+  TimedScope ts("k_conv3x3_wgrad", s);
+  hipLaunchKernelGGL(k_conv3x3_wgrad, dim3(grid), dim3(256), WG_LDS, s, A);
+  FSG_CHECK_LAUNCH("k_conv3x3_wgrad");
+  if (part) {
+    hipLaunchKernelGGL(k_wgrad_reduce, dim3(WG_PART / 64), dim3(256), 0, s, part, grid, cin, dw,
+                       db);
+    FSG_CHECK_LAUNCH("k_wgrad_reduce");
+  }
+  return FSG_OK;
+}
+
 extern "C" int fsg_cnn_conv3x3_wgrad(const void* x, const void* dz, int32_t batch, int32_t h,
                                      int32_t w, int32_t cin, float* dw, float* db,
                                      void* stream) {
-  if (!x || !dz || !dw || !db) return fail(FSG_E_INVALID, "fsg_cnn_conv3x3_wgrad: NULL argument");
-  if (batch <= 0 || h <= 0 || w <= 0 || (cin != 8 && cin != 32))
-    return fail(FSG_E_INVALID, "fsg_cnn_conv3x3_wgrad: bad shape");
-  WgradArgs A{(const u16*)x, (const u16*)dz, dw, db, batch, h, w, cin};
-  const int64_t segs = (int64_t)batch * h * ((w + WG_SEG - 1) / WG_SEG);
-  const int grid = (int)std::min<int64_t>(segs, 1024);
-  hipStream_t s = as_stream(stream);
-  TimedScope ts("k_conv3x3_wgrad", s);
-  hipLaunchKernelGGL(k_conv3x3_wgrad, dim3(grid), dim3(256), 0, s, A);
-  FSG_CHECK_LAUNCH("k_conv3x3_wgrad");
-  return FSG_OK;
+  return wgrad_run(x, dz, batch, h, w, cin, dw, db, nullptr, 0, stream);
+}
+
+extern "C" size_t fsg_cnn_wgrad_workspace_size(int32_t batch, int32_t h, int32_t w) {
+  if (batch <= 0 || h <= 0 || w <= 0) return 0;
+  WgradArgs A{};
+  return (size_t)wgrad_plan(batch, h, w, WG_BLOCKS, A) * WG_PART * sizeof(float);
+}
+
+extern "C" int fsg_cnn_conv3x3_wgrad_ws(const void* x, const void* dz, int32_t batch, int32_t h,
+                                        int32_t w, int32_t cin, float* dw, float* db,
+                                        void* workspace, size_t workspace_bytes, void* stream) {
+  if (!workspace) return fail(FSG_E_WORKSPACE, "fsg_cnn_conv3x3_wgrad: workspace NULL");
+  return wgrad_run(x, dz, batch, h, w, cin, dw, db, (float*)workspace, workspace_bytes, stream);
 }
 
 extern "C" int fsg_cnn_pack(const float* w, int32_t cout, int32_t cin, void* wf, int32_t kpad,

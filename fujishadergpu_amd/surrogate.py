@@ -201,11 +201,13 @@ class Net:
         L = N.lib()
         self.grad.zero_()
         dz = dz_last
+        nb = int(L.fsg_cnn_wgrad_workspace_size(bsz, h, w))
+        ws = torch.empty(nb, dtype=torch.uint8, device=self.device)
         for li in range(len(self.shapes) - 1, -1, -1):
             co, ci = self.shapes[li]
-            N.check(L.fsg_cnn_conv3x3_wgrad(acts[li].data_ptr(), dz.data_ptr(), bsz, h, w, ci,
-                                            self.gw(li).data_ptr(), self.gb(li).data_ptr(),
-                                            _s()))
+            N.check(L.fsg_cnn_conv3x3_wgrad_ws(acts[li].data_ptr(), dz.data_ptr(), bsz, h, w, ci,
+                                               self.gw(li).data_ptr(), self.gb(li).data_ptr(),
+                                               ws.data_ptr(), nb, _s()))
             if li > 0:
                 nd = torch.empty((bsz, h, w, 32), dtype=torch.int16, device=self.device)
                 self._conv(li, dz, h, w, bsz, N.CNN_GELU_GRAD, y=nd, pre_in=pres[li - 1],

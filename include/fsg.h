@@ -598,7 +598,8 @@ int fsg_combine_fields(const float* const* fields, int32_t n, int64_t ld, const 
  *                      layer's pre-activation (backward through conv + GELU).
  * fsg_cnn_conv3x3_wgrad accumulates dw [32][cin][9] and db [32] (f32; zero
  * them first) from the layer input x and the pre-activation gradient dz
- * [..][32] bf16.  fsg_cnn_pack writes the forward and (wt != NULL) backward
+ * [..][32] bf16; the _ws form sums its workgroups' partials through a
+ * workspace of fsg_cnn_wgrad_workspace_size bytes instead of by atomics.  fsg_cnn_pack writes the forward and (wt != NULL) backward
  * bf16 layouts of float32 weights w [cout][cin][3][3].  fsg_cnn_adam is one
  * bias-corrected Adam step on float32 parameters (step counts from 1).
  */
@@ -618,6 +619,10 @@ typedef struct fsg_cnn_conv {
 int fsg_cnn_conv3x3(const fsg_cnn_conv* c, void* stream);
 int fsg_cnn_conv3x3_wgrad(const void* x, const void* dz, int32_t batch, int32_t h, int32_t w,
                           int32_t cin, float* dw, float* db, void* stream);
+size_t fsg_cnn_wgrad_workspace_size(int32_t batch, int32_t h, int32_t w);
+int fsg_cnn_conv3x3_wgrad_ws(const void* x, const void* dz, int32_t batch, int32_t h, int32_t w,
+                             int32_t cin, float* dw, float* db, void* workspace,
+                             size_t workspace_bytes, void* stream);
 int fsg_cnn_pack(const float* w, int32_t cout, int32_t cin, void* wf, int32_t kpad, void* wt,
                  int32_t kpad_t, void* stream);
 int fsg_cnn_adam(float* p, const float* g, float* m, float* v, int32_t n, float lr,

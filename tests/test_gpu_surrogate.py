@@ -108,6 +108,45 @@ def test_backward_matches_oracle_gradients(cuda):
             assert cos > 0.999 and rel < 0.05, f"layer {li} d{name}: cos {cos:.5f} rel {rel:.3f}"
 
 
+@pytest.mark.parametrize("cin", [8, 32])
+@pytest.mark.parametrize("bsz,h,w", [(1, 1, 1), (1, 5, 16), (2, 4, 17), (1, 3, 96), (1, 7, 97),
+                                     (3, 9, 203), (40, 60, 33)])
+def test_wgrad_at_strip_and_row_group_edges(cuda, cin, bsz, h, w):
+    """Both weight-gradient entry points against float64 sums over one-pixel images, strips
+    of one and of several widths, partial row groups, and more tasks than blocks.  Float32
+    sums of n products are off by at most n 2^-24 times the sum of their magnitudes."""
+    from fujishadergpu_amd import _native as N
+    g = torch.Generator(device=cuda).manual_seed(7)
+    x = torch.randn((bsz, h, w, cin), generator=g, device=cuda).to(torch.bfloat16)
+    dz = torch.randn((bsz, h, w, 32), generator=g, device=cuda).to(torch.bfloat16)
+    L, s = N.lib(), torch.cuda.current_stream().cuda_stream
+    nb = int(L.fsg_cnn_wgrad_workspace_size(bsz, h, w))
+    ws = torch.empty(nb, dtype=torch.uint8, device=cuda)
+    xp = torch.nn.functional.pad(x.double(), (0, 0, 1, 1, 1, 1))
+    z = dz.double().reshape(-1, 32)
+    bound = bsz * h * w * 2.0 ** -24
+    for entry in ("atomic", "workspace"):
+        dw = torch.full((32, cin, 9), 0.5, device=cuda)      # accumulated onto
+        db = torch.full((32,), -0.25, device=cuda)
+        if entry == "atomic":
+            N.check(L.fsg_cnn_conv3x3_wgrad(x.data_ptr(), dz.data_ptr(), bsz, h, w, cin,
+                                            dw.data_ptr(), db.data_ptr(), s))
+        else:
+            N.check(L.fsg_cnn_conv3x3_wgrad_ws(x.data_ptr(), dz.data_ptr(), bsz, h, w, cin,
+                                               dw.data_ptr(), db.data_ptr(), ws.data_ptr(), nb,
+                                               s))
+        for tap in range(9):
+            xs = xp[:, tap // 3:tap // 3 + h, tap % 3:tap % 3 + w].reshape(-1, cin)
+            ref, mag = z.T @ xs + 0.5, z.abs().T @ xs.abs() + 0.5
+            assert bool(((dw[:, :, tap].double() - ref).abs() <= bound * mag + 1e-7).all()), tap
+        assert bool(((db.double() - (z.sum(0) - 0.25)).abs()
+                     <= bound * z.abs().sum(0) + 1e-7).all())
+    with pytest.raises(N.FsgError):
+        N.check(L.fsg_cnn_conv3x3_wgrad_ws(x.data_ptr(), dz.data_ptr(), bsz, h, w, cin,
+                                           dw.data_ptr(), db.data_ptr(), ws.data_ptr(), nb - 1,
+                                           s))
+
+
 @pytest.mark.parametrize("f", [8, 4, 16])
 def test_compose_and_detail_label_match_the_oracle(cuda, f):
     from fujishadergpu_amd import _native as N
