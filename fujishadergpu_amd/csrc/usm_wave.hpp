@@ -89,75 +89,6 @@ __device__ __forceinline__ double bits_f64(int lo, int hi) {
   return __builtin_bit_cast(double, ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
 }
 
-// The epilogue of four consecutive outputs, branch-free per value (the
-// uniform choices are made once per call).  post: apply_post's arithmetic;
-// store: store_out's (clip, quantisation, NaN -> 0 for integer outputs).
-__device__ __forceinline__ float post_value(const PostK& p, float v) {
-  if (p.kind == 1) {
-    const float q = v / p.sc;                     // NaN stays NaN
-    return p.zero ? (isnan(v) ? v : 0.0f) : q;
-  }
-  if (p.kind == 2) {
-    const float q = (v - p.lo) / p.sc;
-    return isnan(q) ? q : fmaxf(q, 0.0f);
-  }
-  return v;
-}
-
-__device__ __forceinline__ float dn_value(const OutDev& o, float v) {
-  float t = o.a * v;
-  t = t + o.b;
-  t = rintf(t);
-  t = fminf(fmaxf(t, o.dn_min), o.dn_max);
-  return isfinite(v) ? t : 0.0f;
-}
-
-// Values m_lo .. m_hi - 1 of four consecutive output columns starting at
-// region column c, row r.  full4: every lane's group is all-or-nothing
-// (uniform), so a lane with outputs writes one vector.
-__device__ __forceinline__ void store_out4(const OutDev& o, int r, int c, const float v[4],
-                                           int m_lo, int m_hi, bool full4) {
-  float w[4];
-#pragma unroll
-  for (int m = 0; m < 4; m++) w[m] = v[m];
-  if (o.clip01) {
-#pragma unroll
-    for (int m = 0; m < 4; m++) w[m] = isnan(w[m]) ? w[m] : fminf(fmaxf(w[m], 0.0f), 1.0f);
-  }
-  const int64_t off = (int64_t)r * o.ld + c;
-  if (o.dtype == FSG_OUT_F32) {
-    float* p = (float*)o.data + off;
-    if (full4) {  // one 16-byte store (dword-aligned)
-      const float4 q = make_float4(w[0], w[1], w[2], w[3]);
-      __builtin_memcpy(p, &q, sizeof(q));
-    } else {
-#pragma unroll
-      for (int m = 0; m < 4; m++)
-        if (m >= m_lo && m < m_hi) p[m] = w[m];
-    }
-    return;
-  }
-  float d[4];
-#pragma unroll
-  for (int m = 0; m < 4; m++) d[m] = dn_value(o, w[m]);
-  if (o.dtype == FSG_OUT_I16) {
-    int16_t* p = (int16_t*)o.data + off;
-#pragma unroll
-    for (int m = 0; m < 4; m++)
-      if (m >= m_lo && m < m_hi) p[m] = (int16_t)(int)d[m];
-  } else {
-    uint8_t* p = (uint8_t*)o.data + off;
-    if (full4 && (((uintptr_t)o.data | (uintptr_t)o.ld) & 3) == 0) {
-      *(uint32_t*)p = (uint32_t)(int)d[0] | ((uint32_t)(int)d[1] << 8) |
-                      ((uint32_t)(int)d[2] << 16) | ((uint32_t)(int)d[3] << 24);
-    } else {
-#pragma unroll
-      for (int m = 0; m < 4; m++)
-        if (m >= m_lo && m < m_hi) p[m] = (uint8_t)(int)d[m];
-    }
-  }
-}
-
 // One SW x SH block of the region.  P: this wave's LDS prefix buffer (4 *
 // WAVE_PB doubles, one radius at a time).  Hc: its LDS copy of the float64
 // coarse-row values of each source, [NS][2][WAVE_NC] (lane t uses columns

@@ -661,3 +661,43 @@ def test_wave_kernel_equals_the_workgroup_kernel(cuda, radii, weights, px, shape
     exp = ref.topousm_direct(dem.numpy(), **kw)[r0:r0 + rh, c0:c0 + rw]
     mx, _ = _cmp("topousm/wave", b32, exp, 2e-5)
     print("radii", radii, "max |d| vs oracle", mx, flush=True)
+
+
+@pytest.mark.parametrize("h,w,dist,n_dirs,typ", [
+    (384, 384, 50, 16, "positive"), (2304, 64, 64, 8, "negative"), (1153, 128, 8, 33, "positive"),
+    (390, 389, 68, 3, "negative"), (385, 383, 69, 5, "positive"), (600, 257, 3, 1, "positive")])
+def test_openness_tiles_equal_the_pointwise_rays(cuda, h, w, dist, n_dirs, typ):
+    """Regions large enough for the tiles staged in LDS (the reach at their limit and past
+    it, one column panel and ragged ones, voids and the window's edges) against the
+    point entry point, which samples memory pixel by pixel: the same bits."""
+    from fujishadergpu_amd import ops, synth
+    from fujishadergpu_amd.algorithms import openness_table
+    dem = synth.fbm(h + 40, w + 30, 0.8, 900.0, seed=5, device="cuda")
+    synth.apply_discs(dem, [(h // 2, w // 3, 41), (30, w - 5, 20), (h, 12, 9)], float("nan"))
+    win = dem[7:7 + h + 24, 3:3 + w + 11]                   # an odd row start, a halo
+    reg = ops.region(9, 5, h, w)
+    table = openness_table(n_dirs, dist, 5.0)
+    out = torch.empty((h, w), dtype=torch.float32, device=cuda)
+    ops.openness(win, reg, table=table, openness_type=typ, out=ops.output(out))
+    rr, cc = torch.meshgrid(torch.arange(h), torch.arange(w), indexing="ij")
+    pts = torch.stack([rr.reshape(-1) + 9, cc.reshape(-1) + 5], 1).to(torch.int32).to(cuda)
+    ref = ops.openness_points(win, pts, table=table, openness_type=typ, raw_degrees=False)
+    assert torch.equal(out.view(-1).view(torch.int32), ref.view(torch.int32))
+
+
+@pytest.mark.parametrize("h,w,samples,radius,px", [
+    (384, 384, 16, 10.0, 10.0), (500, 301, 7, 33.0, 2.0), (1160, 129, 1, 64.0, 5.0),
+    (385, 383, 61, 3.0, 1.0)])
+def test_ambient_occlusion_tiles_match_the_oracle(cuda, h, w, samples, radius, px):
+    """AO from tiles staged in LDS: full and partial sample groups, runs longer than one
+    word of groups allows, a reach at the limit, voids, ragged strips of the smoothing."""
+    from fujishadergpu_amd import synth
+    from fujishadergpu_amd.algorithms import ALGORITHMS
+    dem = synth.fbm(h, w, 0.7, 400.0, seed=6, device="cuda")
+    synth.apply_discs(dem, [(h // 2, w // 3, 21), (30, w - 5, 20)], float("nan"))
+    got = ALGORITHMS["ambient_occlusion"].process(dem, num_samples=samples, radius=radius,
+                                                  pixel_size=px).cpu().numpy()
+    want = ref.ambient_occlusion(dem.cpu().numpy(), num_samples=samples, radius=radius,
+                                 pixel_size=px)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.nanmax(np.abs(got - want)) < 1e-5
