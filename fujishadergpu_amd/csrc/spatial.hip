@@ -45,17 +45,25 @@ struct PadSrc {
   }
 };
 
-// The NaN-aware Gaussian runs as two LDS-tiled passes over 64 x 64 output
-// tiles.  Each of the 4 waves of a block owns GN_M consecutive outputs along
-// the filter axis for 64 lines across it, so one sample loaded from LDS into
-// a register serves GN_M outputs: the pair (x[-d], x[+d]) of output m at
-// distance d is x[m - d], x[m + d], and a block of GN_M distances reads two
-// register windows of 2 GN_M - 1 samples that slide by GN_M per block.  Every
-// output still accumulates in scipy's symmetric order, in float64: the
-// centre, then acc + (x[-d] + x[+d]) * g[d] for d = r .. 1, each operation
-// rounded on its own (the library builds with -ffp-contract=off).
-constexpr int GN_T = 64;   // output tile edge
-constexpr int GN_M = 16;   // outputs per lane along the filter axis (4 waves x 16 = 64)
+// The NaN-aware Gaussian runs as two LDS-tiled passes over output tiles of 128 along
+// the filter axis and 64 across it, each a product with a band matrix in float64 on the matrix cores
+// (v_mfma_f64_16x16x4_f64: lane l holds A[l % 16][l / 16], B[l / 16][l % 16] and,
+// in entry e, D[l / 16 + 4 e][l % 16]): T[y][k] = g[|k - y - r|] over the 16 + 2 r
+// samples that 16 outputs reach, zero outside the band, so the LDS span past a
+// window of taps must be finite.  Sums stay float64; only their order is the
+// matrix cores', not scipy's, which the float32 rounding after each axis hides
+// but for near-ties.  A tile whose span holds an infinity takes gn_slow, scipy's
+// order tap by tap: zero weights must not meet it.
+// Bound: float64 MFMA issue, (16 + 2 r) / 4 instructions of 64 cycles per 16 x 16
+// outputs, for the wide filters (r = 64: 144 of 129 taps); memory for r <= 16.
+// As VALU sums (3 operations per pair of taps) the passes took 147 and 164 us on
+// average over an 8192^2 hillshade job's 17 windows; now 97 and 98.
+// A wave owns 32 outputs along the axis as two groups of 16: the second group's
+// band is the first's 16 samples later, so a sample's LDS read and conversion
+// serve eight products.
+constexpr int GN_T = 64;   // tile extent across the filter axis
+constexpr int GN_L = 128;  // ... along it
+typedef double d4 __attribute__((ext_vector_type(4)));
 
 // sample as the accumulation sees it: 0 plain, 1 NaN -> 0, 2 validity (0 / 1)
 template <int MODE>
@@ -65,177 +73,290 @@ __device__ __forceinline__ double gn_val(float f) {
   else return isnan(f) ? 0.0 : 1.0;
 }
 
-// acc[m] = sum_k g[|k|] v(s[(m + k) ST]), k in [-r, r], in the order above.
-// s points at the lane's first output; the LDS line holds r samples before
-// it and r + GN_M - 1 after it.
-template <int MODE, int ST>
-__device__ __forceinline__ void gn_line(const float* s, const GaussW& G, double (&acc)[GN_M]) {
-  const double g0 = G.g[0];
+// The band's weights: T[t] = g[|t - 15 - r|] (0 past r), so that output y and
+// sample k take T[k - y + 15].  n <= 512 entries, two per thread: the loads are
+// issued (gn_band) ahead of the tile's and stored (put) after them.
+struct GnBand {
+  double v[2];
+  __device__ __forceinline__ void get(const GaussW& G) {
 #pragma unroll
-  for (int m = 0; m < GN_M; m++) acc[m] = gn_val<MODE>(s[m * ST]) * g0;
-  int d = G.r;
-  for (; d % GN_M != 0; d--) {   // the top r mod GN_M distances one at a time
-    const double g = G.g[d];
-#pragma unroll
-    for (int m = 0; m < GN_M; m++)
-      acc[m] = acc[m] + (gn_val<MODE>(s[(m - d) * ST]) + gn_val<MODE>(s[(m + d) * ST])) * g;
-  }
-  if (d == 0) return;
-  // distances d .. d - GN_M + 1: L[k] = x[k - d], R[k] = x[k + d - GN_M + 1]
-  double L[2 * GN_M - 1], R[2 * GN_M - 1];
-#pragma unroll
-  for (int k = 0; k < 2 * GN_M - 1; k++) {
-    L[k] = gn_val<MODE>(s[(k - d) * ST]);
-    R[k] = gn_val<MODE>(s[(k + d - (GN_M - 1)) * ST]);
-  }
-  for (;;) {
-#pragma unroll
-    for (int dd = 0; dd < GN_M; dd++) {
-      const double g = G.g[d - dd];
-#pragma unroll
-      for (int m = 0; m < GN_M; m++) acc[m] = acc[m] + (L[m + dd] + R[m - dd + GN_M - 1]) * g;
+    for (int u = 0; u < 2; u++) {
+      const int d = abs((int)threadIdx.x + 256 * u - 15 - G.r);
+      v[u] = d <= G.r ? G.g[min(d, GN_MAX_R)] : 0.0;
     }
-    d -= GN_M;
-    if (d == 0) break;
-#pragma unroll
-    for (int k = 0; k < GN_M - 1; k++) L[k] = L[k + GN_M];
-#pragma unroll
-    for (int k = GN_M - 1; k < 2 * GN_M - 1; k++) L[k] = gn_val<MODE>(s[(k - d) * ST]);
-#pragma unroll
-    for (int k = 2 * GN_M - 2; k >= GN_M; k--) R[k] = R[k - GN_M];
-#pragma unroll
-    for (int k = 0; k < GN_M; k++) R[k] = gn_val<MODE>(s[(k + d - (GN_M - 1)) * ST]);
   }
+  __device__ __forceinline__ void put(double* T, int n) const {
+    if ((int)threadIdx.x < n) T[threadIdx.x] = v[0];
+    if ((int)threadIdx.x + 256 < n) T[threadIdx.x + 256] = v[1];
+  }
+};
+
+// One output in scipy's symmetric order: the centre, then acc + (x[-d] + x[+d]) *
+// g[d] for d = r .. 1, each operation rounded on its own.  T: the band.
+template <int MODE>
+__device__ __forceinline__ double gn_slow(const float* s, int st, const double* T, int r) {
+  const double* g = T + 15 + r;
+  double acc = gn_val<MODE>(s[0]) * g[0];
+#pragma unroll 1
+  for (int d = r; d >= 1; d--)
+    acc = acc + (gn_val<MODE>(s[-d * st]) + gn_val<MODE>(s[d * st])) * g[d];
+  return acc;
 }
+
+__host__ __device__ inline int gn_ksteps(int r, int step) { return (16 + 2 * r + step - 1) / step; }
 
 // Pass 0 (axis 0) over the padded extent: tv = f32(sum g * where(nan, 0, x)),
 // tw = f32(sum g * valid).  A tile whose input span holds no NaN has tw =
-// f32(wsum) everywhere, wsum being the same accumulation over all-valid
-// samples (computed on the host by the same operation sequence).
-// LDS: (64 + 2r) rows x 64 columns.
-__global__ __launch_bounds__(256, 2) void k_gauss_nan_rows(PadSrc S, GaussW G,
-                                                           float* __restrict__ tv,
-                                                           float* __restrict__ tw, int64_t ldt,
-                                                           float wconst) {
-  extern __shared__ float gl[];
-  const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
-  const int hp = S.h + 2 * S.pad, wp = S.w + 2 * S.pad;
-  const int tx0 = blockIdx.x * GN_T, ty0 = blockIdx.y * GN_T;
-  const int nrow = GN_T + 2 * G.r;
-  const int pc = min(tx0 + lane, wp - 1);
-  bool nan = false;
-  // staging in batches of 8 rows per wave (8 loads in flight per lane)
-  for (int i0 = q; i0 < nrow; i0 += 32) {
-    float v[8];
+// f32(wsum) everywhere, wsum being the same accumulation over all-valid samples
+// (on the host): it writes no tw but the mark -1 at its first pixel.
+// LDS: the band, then 112 + 4 n_ks rows of 64 columns.  A lane's sample of the four
+// column tiles is one 16-byte read: tile n has the columns 4 j + n, so a lane
+// holds four consecutive outputs of a row.
+template <int MODE>
+__device__ __forceinline__ void gn_rows_mma(const float* s, const double* T, int n_ks, int lane,
+                                            d4 (&acc)[2][4]) {
+  const int k = lane >> 4, j = lane & 15;
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
-      const int i = i0 + 4 * u;
-      v[u] = i < nrow ? S.at(ty0 - G.r + i, pc) : 0.0f;
+  for (int n = 0; n < 4; n++) acc[0][n] = acc[1][n] = d4{0.0, 0.0, 0.0, 0.0};
+  const float* p = s + k * GN_T + 4 * j;
+  const double* tp = T + k - j + 15;
+  auto step = [&](int ks, bool g0, bool g1) {
+    const float4 v = *(const float4*)(p + 4 * ks * GN_T);
+    const double x[4] = {gn_val<MODE>(v.x), gn_val<MODE>(v.y), gn_val<MODE>(v.z),
+                         gn_val<MODE>(v.w)};
+    if (g0) {
+      const double a = tp[4 * ks];
+#pragma unroll
+      for (int n = 0; n < 4; n++)
+        acc[0][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, x[n], acc[0][n], 0, 0, 0);
+    }
+    if (g1) {
+      const double a = tp[4 * ks - 16];
+#pragma unroll
+      for (int n = 0; n < 4; n++)
+        acc[1][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, x[n], acc[1][n], 0, 0, 0);
+    }
+  };
+#pragma unroll 2
+  for (int ks = 0; ks < 4; ks++) step(ks, true, false);
+#pragma unroll 2
+  for (int ks = 4; ks < n_ks; ks++) step(ks, true, true);
+#pragma unroll 2
+  for (int ks = n_ks; ks < n_ks + 4; ks++) step(ks, false, true);
+}
+
+__global__ __launch_bounds__(256, 2) void k_gauss_nan_rows(PadSrc S, GaussW G, int n_ks,
+                                                        float* __restrict__ tv,
+                                                        float* __restrict__ tw, int64_t ldt) {
+  extern __shared__ __attribute__((aligned(16))) double gband[];
+  const int n_band = (4 * n_ks + 16 + 1) & ~1;
+  float* const gl = (float*)(gband + n_band);
+  const int lane = threadIdx.x & 63;
+  const int q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hp = S.h + 2 * S.pad, wp = S.w + 2 * S.pad;
+  const int tx0 = blockIdx.x * GN_T, ty0 = blockIdx.y * GN_L;
+  const int nrow = GN_L + 2 * G.r, npad = 112 + 4 * n_ks;
+  GnBand B;
+  B.get(G);
+  bool nan = false, inf = false;
+  // staging in batches of 32 rows per wave: with two blocks a CU, what a batch
+  // waits for memory is hidden by little else
+  const int wr0 = ty0 - G.r - S.pad, wc0 = tx0 - S.pad;   // window row and column of (0, 0)
+  const bool inside = wr0 >= 0 && wr0 + nrow <= S.h && wc0 >= 0 && wc0 + GN_T <= S.w;
+  const int pc = min(tx0 + lane, wp - 1);
+  const float* const base = inside ? S.p + (int64_t)wr0 * S.ld + wc0 : S.p;
+  const int wc = inside ? lane : sym(pc - S.pad, S.w);
+  constexpr int GN_B = 32;
+  for (int i0 = q; i0 < npad; i0 += 4 * GN_B) {
+    float v[GN_B];
+#pragma unroll
+    for (int u = 0; u < GN_B; u++) {
+      const int i = min(i0 + 4 * u, nrow - 1);
+      const int row = inside ? i : sym(min(max(ty0 - G.r + i, 0), hp - 1) - S.pad, S.h);
+      v[u] = (base + (int64_t)row * S.ld)[wc];
     }
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
+    for (int u = 0; u < GN_B; u++) {
       const int i = i0 + 4 * u;
-      if (i < nrow) {
-        gl[i * GN_T + lane] = v[u];
-        nan |= isnan(v[u]);
+      if (i >= npad) break;
+      const float x = i < nrow ? v[u] : 0.0f;
+      gl[i * GN_T + lane] = x;
+      nan |= isnan(x);
+      inf |= isinf(x);
+    }
+  }
+  B.put(gband, n_band);
+  const bool any_nan = __syncthreads_or(nan);
+  const bool any_inf = __syncthreads_or(inf);
+  const int j = lane & 15;
+  // entry e of the lane's groups: row y0 + 4 e, columns x .. x + 3
+  const int x = tx0 + 4 * j, y0 = ty0 + q * 32 + (lane >> 4);
+  auto store = [&](float* dst, const d4 (&acc)[2][4]) {
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const int y = y0 + 4 * e;
+      if (y >= hp) break;
+      const d4 (&a)[4] = acc[e >> 2];
+      const float v[4] = {(float)a[0][e & 3], (float)a[1][e & 3], (float)a[2][e & 3],
+                          (float)a[3][e & 3]};
+      float* o = dst + (int64_t)y * ldt + x;
+      if (x + 3 < wp) {
+        __builtin_memcpy(o, v, 16);
+      } else {
+#pragma unroll
+        for (int n = 0; n < 3; n++)
+          if (x + n < wp) o[n] = v[n];
       }
     }
-  }
-  const bool any_nan = __syncthreads_or(nan);
-  const float* s = gl + (q * GN_M + G.r) * GN_T + lane;
-  const int x = tx0 + lane;
-  const int y0 = ty0 + q * GN_M;
-  const int nm = x < wp ? min(GN_M, hp - y0) : 0;   // rows this lane stores
-  double acc[GN_M];
-  if (any_nan) gn_line<1, GN_T>(s, G, acc);
-  else gn_line<0, GN_T>(s, G, acc);
-#pragma unroll
-  for (int m = 0; m < GN_M; m++)
-    if (m < nm) tv[(int64_t)(y0 + m) * ldt + x] = (float)acc[m];
-  if (!any_nan) {
-#pragma unroll
-    for (int m = 0; m < GN_M; m++)
-      if (m < nm) tw[(int64_t)(y0 + m) * ldt + x] = wconst;
+  };
+  if (any_inf) {
+#pragma unroll 1
+    for (int m = 0; m < 32; m++) {
+      const int y = ty0 + q * 32 + m;
+      if (y >= hp || tx0 + lane >= wp) break;
+      const float* s = gl + (q * 32 + m + G.r) * GN_T + lane;
+      const int64_t o = (int64_t)y * ldt + tx0 + lane;
+      tv[o] = (float)gn_slow<1>(s, GN_T, gband, G.r);
+      tw[o] = (float)gn_slow<2>(s, GN_T, gband, G.r);
+    }
     return;
   }
-  gn_line<2, GN_T>(s, G, acc);
-#pragma unroll
-  for (int m = 0; m < GN_M; m++)
-    if (m < nm) tw[(int64_t)(y0 + m) * ldt + x] = (float)acc[m];
+  const float* s = gl + q * 32 * GN_T;
+  d4 acc[2][4];
+  if (!any_nan) {
+    gn_rows_mma<0>(s, gband, n_ks, lane, acc);
+    store(tv, acc);
+    if (threadIdx.x == 0) tw[(int64_t)ty0 * ldt + tx0] = -1.0f;
+    return;
+  }
+  gn_rows_mma<1>(s, gband, n_ks, lane, acc);
+  store(tv, acc);
+  gn_rows_mma<2>(s, gband, n_ks, lane, acc);
+  store(tw, acc);
 }
 
 // Pass 1 (axis 1, 'nearest' along the padded rows) and where(sw > 0, sv / sw,
-// 0) in float32.  A tile whose tw span is all f32(wsum) divides by the
-// constant f32 of that accumulation (wdiv, from the host).  LDS: 64 rows x
-// (64 + 2r + 1) columns (odd pitch: lanes walk rows without bank conflicts),
-// reused for tw, tv and the transposed output tile.
+// 0) in float32.  Where every tile of the span is marked as without NaN, sw is
+// the constant f32 of that accumulation (wdiv, from the host).
+// LDS: the band, then 64 rows of P floats (P = 4 mod 64: the 16 rows of a 16-byte
+// read spread over the banks) for the 112 + 16 n_ks samples, those past 128 + 2 r
+// zero.  A step takes 16 samples: lane group k = l / 16 reads samples 4 k .. 4 k +
+// 3 of its row at once, and MFMA t of the step takes sample 4 k + t.
+__device__ __forceinline__ void gn_cols_mma(const float* s, int P, const double* T, int n_ks,
+                                            int lane, d4 (&acc)[2][4]) {
+  const int k = lane >> 4, j = lane & 15;
+#pragma unroll
+  for (int m = 0; m < 4; m++) acc[0][m] = acc[1][m] = d4{0.0, 0.0, 0.0, 0.0};
+  const float* p = s + j * P + 4 * k;
+  const double* tp = T + 4 * k - j + 15;
+  double b[4] = {0.0, 0.0, 0.0, 0.0};   // the band of the step, which is the second
+                                        // group's in the step after
+  auto step = [&](int ks, bool g0, bool g1) {
+    double c[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) c[t] = g0 ? tp[16 * ks + t] : 0.0;
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+      const float4 v = *(const float4*)(p + 16 * m * P + 16 * ks);
+      const double x[4] = {(double)v.x, (double)v.y, (double)v.z, (double)v.w};
+#pragma unroll
+      for (int t = 0; t < 4; t++) {
+        if (g0) acc[0][m] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[t], c[t], acc[0][m], 0, 0, 0);
+        if (g1) acc[1][m] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[t], b[t], acc[1][m], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < 4; t++) b[t] = c[t];
+  };
+  step(0, true, false);
+#pragma unroll 1
+  for (int ks = 1; ks < n_ks; ks++) step(ks, true, true);
+  step(n_ks, false, true);
+}
+
 __global__ __launch_bounds__(256, 2) void k_gauss_nan_cols(const float* __restrict__ tv,
                                                         const float* __restrict__ tw, int64_t ldt,
-                                                        int hp, int wp, GaussW G,
+                                                        int hp, int wp, GaussW G, int n_ks, int P,
                                                         float* __restrict__ out, int64_t ldo,
                                                         float wconst, float wdiv) {
-  extern __shared__ float gl[];
-  const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
-  const int tx0 = blockIdx.x * GN_T, ty0 = blockIdx.y * GN_T;
-  const int ncol = GN_T + 2 * G.r, P = ncol + 1;
-  // staging: column chunks of 64, each in batches of 8 rows per wave (8 loads in flight)
-  auto stage = [&](const float* src) {
-    bool off = false;
-    for (int c = 0; c < ncol; c += 64) {
-      const int j = c + lane;
-      const bool jok = j < ncol;
-      const int col = min(max(tx0 - G.r + j, 0), wp - 1);
+  extern __shared__ __attribute__((aligned(16))) double gband[];
+  const int n_band = (16 * n_ks + 16 + 1) & ~1;
+  float* const gl = (float*)(gband + n_band);
+  const int lane = threadIdx.x & 63;
+  const int q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tx0 = blockIdx.x * GN_L, ty0 = blockIdx.y * GN_T;
+  const int ncol = GN_L + 2 * G.r, npad = 112 + 16 * n_ks;
+  const float* const mark = tw + (int64_t)(ty0 / GN_L * GN_L) * ldt;   // of this row of tiles
+  GnBand B;
+  B.get(G);
+  // the marks of the tiles that the span touches
+  const int t_lo = max(tx0 - G.r, 0) / GN_T, t_hi = min(tx0 + GN_L - 1 + G.r, wp - 1) / GN_T;
+  bool varied = false;
+  for (int t = t_lo; t <= t_hi; t++) varied |= mark[t * GN_T] != -1.0f;
+  // staging: two 64-column pieces of a wave's 16 rows in flight; weights: a marked
+  // tile's tw is wconst
+  auto stage = [&](const float* src, bool weights) {
+    bool odd = false;
+    for (int c = 0; c < npad; c += 128) {
+      float v[2][16];
 #pragma unroll
-      for (int k0 = 0; k0 < GN_T / 4; k0 += 8) {
-        float v[8];
+      for (int h = 0; h < 2; h++) {
+        const int col = min(max(tx0 - G.r + c + 64 * h + lane, 0), wp - 1);
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-          const int i = q + 4 * (k0 + u);
-          v[u] = jok ? src[(int64_t)min(ty0 + i, hp - 1) * ldt + col] : 0.0f;
-        }
+        for (int u = 0; u < 16; u++)
+          v[h][u] = (src + (int64_t)min(ty0 + q + 4 * u, hp - 1) * ldt)[col];
+      }
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-          const int i = q + 4 * (k0 + u);
-          if (jok) {
-            gl[i * P + j] = v[u];
-            off |= __float_as_uint(v[u]) != __float_as_uint(wconst);
-          }
+      for (int h = 0; h < 2; h++) {
+        const int j = c + 64 * h + lane;
+        const int col = min(max(tx0 - G.r + j, 0), wp - 1);
+        const bool marked = weights && mark[col / GN_T * GN_T] == -1.0f;
+        if (j >= npad) continue;
+#pragma unroll
+        for (int u = 0; u < 16; u++) {
+          const float x = j >= ncol ? 0.0f : marked ? wconst : v[h][u];
+          gl[(q + 4 * u) * P + j] = x;
+          odd |= !isfinite(x);
         }
       }
     }
-    return off;
+    return odd;
   };
-  const float* s = gl + lane * P + q * GN_M + G.r;
-  double acc[GN_M];
-  float fw[GN_M], fo[GN_M];
-  const bool varied = __syncthreads_or(stage(tw));
+  // entry e of acc[g][m]: row ty0 + 16 m + l / 16 + 4 e, column tx0 + 32 q + 16 g + l % 16
+  const float* s = gl + q * 32;
+  d4 acc[2][4];
+  float fw[2][4][4];
+  B.put(gband, n_band);
   if (varied) {
-    gn_line<0, 1>(s, G, acc);
-#pragma unroll
-    for (int m = 0; m < GN_M; m++) fw[m] = (float)acc[m];
-  } else {
-#pragma unroll
-    for (int m = 0; m < GN_M; m++) fw[m] = wdiv;
+    stage(tw, true);
+    __syncthreads();
+    gn_cols_mma(s, P, gband, n_ks, lane, acc);
+    __syncthreads();
   }
-  __syncthreads();
-  stage(tv);
-  __syncthreads();
-  gn_line<0, 1>(s, G, acc);
 #pragma unroll
-  for (int m = 0; m < GN_M; m++) {
-    const float v = (float)acc[m];
-    fo[m] = fw[m] > 0.0f ? v / fw[m] : 0.0f;
-  }
-  __syncthreads();
+  for (int g = 0; g < 2; g++)
 #pragma unroll
-  for (int m = 0; m < GN_M; m++) gl[lane * (GN_T + 1) + q * GN_M + m] = fo[m];
-  __syncthreads();
-  const int x = tx0 + lane;
-  if (x >= wp) return;
-  for (int i = q; i < GN_T; i += 4) {
-    const int y = ty0 + i;
-    if (y < hp) out[(int64_t)y * ldo + x] = gl[i * (GN_T + 1) + lane];
-  }
+    for (int m = 0; m < 4; m++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) fw[g][m][e] = varied ? (float)acc[g][m][e] : wdiv;
+  const bool odd = __syncthreads_or(stage(tv, false));
+  if (!odd) gn_cols_mma(s, P, gband, n_ks, lane, acc);
+#pragma unroll
+  for (int g = 0; g < 2; g++)
+#pragma unroll
+    for (int m = 0; m < 4; m++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int i = 16 * m + (lane >> 4) + 4 * e, c = 32 * q + 16 * g + (lane & 15);
+        float v;
+        if (odd)
+          v = (float)gn_slow<0>(gl + i * P + c + G.r, 1, gband, G.r);
+        else
+          v = (float)acc[g][m][e];
+        const float f = fw[g][m][e];
+        if (tx0 + c < wp && ty0 + i < hp)
+          out[(int64_t)(ty0 + i) * ldo + tx0 + c] = f > 0.0f ? v / f : 0.0f;
+      }
 }
 
 __global__ void k_pad_sym(PadSrc S, float* __restrict__ out, int64_t ldo) {
@@ -391,15 +512,19 @@ extern "C" int fsg_gaussian_nan(const fsg_window* src, int32_t pad, double sigma
   float* tw = (float*)((char*)workspace + need / 2);
   hipStream_t s = as_stream(stream);
   PadSrc S{src->data, src->ld, src->h, src->w, pad};
-  const dim3 grid((wp + GN_T - 1) / GN_T, (hp + GN_T - 1) / GN_T);
-  const size_t lds_r = sizeof(float) * (GN_T + 2 * G.r) * GN_T;
-  const size_t lds_c = sizeof(float) * GN_T * (GN_T + 2 * G.r + 1);
+  const dim3 grid_r((wp + GN_T - 1) / GN_T, (hp + GN_L - 1) / GN_L);
+  const dim3 grid_c((wp + GN_L - 1) / GN_L, (hp + GN_T - 1) / GN_T);
+  const int ks_r = gn_ksteps(G.r, 4), ks_c = gn_ksteps(G.r, 16);
+  const int P = (112 + 16 * ks_c + 63) / 64 * 64 + 4;
+  const size_t lds_r =
+      sizeof(double) * ((4 * ks_r + 17) & ~1) + sizeof(float) * (112 + 4 * ks_r) * GN_T;
+  const size_t lds_c = sizeof(double) * ((16 * ks_c + 17) & ~1) + sizeof(float) * GN_T * P;
   TimedScope ts("k_gauss_nan", s);
-  hipLaunchKernelGGL(k_gauss_nan_rows, grid, dim3(256), lds_r, s, S, G, tv, tw, (int64_t)wp,
-                     wconst);
+  hipLaunchKernelGGL(k_gauss_nan_rows, grid_r, dim3(256), lds_r, s, S, G, ks_r, tv, tw,
+                     (int64_t)wp);
   FSG_CHECK_LAUNCH("k_gauss_nan_rows");
-  hipLaunchKernelGGL(k_gauss_nan_cols, grid, dim3(256), lds_c, s, tv, tw, (int64_t)wp, hp, wp, G,
-                     out, ldo, wconst, wdiv);
+  hipLaunchKernelGGL(k_gauss_nan_cols, grid_c, dim3(256), lds_c, s, tv, tw, (int64_t)wp, hp, wp, G,
+                     ks_c, P, out, ldo, wconst, wdiv);
   FSG_CHECK_LAUNCH("k_gauss_nan_cols");
   return FSG_OK;
 }

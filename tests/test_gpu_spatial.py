@@ -274,3 +274,41 @@ def test_scheduler_stack_with_the_overview_and_uint8(cuda):
     dn = ref.quantize(f32.cpu().numpy(), qp["a_coef"], qp["b_coef"], qp["dn_min"], qp["dn_max"],
                       "uint8")
     assert np.array_equal(out.cpu().numpy(), dn)
+
+
+@pytest.mark.parametrize("h,w,pad,sigma", [(1, 1, 0, 0.5), (64, 128, 0, 1.0), (129, 65, 3, 4.0),
+                                           (300, 257, 17, 10.25), (140, 513, 60, 40.0)])
+@pytest.mark.parametrize("special", ["none", "nan", "inf", "all_nan"])
+def test_gaussian_band_products_against_float64(cuda, h, w, pad, sigma, special):
+    """The band products at one-pixel, one-tile and ragged extents, for the fewest and the
+    most taps, against float64 sums: one float32 rounding per axis and of the quotient
+    (1.8e-7 relative of the largest weight sum).  An infinity reaches exactly the outputs
+    whose taps cover it."""
+    from fujishadergpu_amd import spatial
+    dem = _dem(max(h, 8), max(w, 8), 51)[:h, :w].contiguous() + 100.0
+    if special == "nan":
+        dem[h // 3:h // 3 + 9, w // 4:w // 4 + 30] = float("nan")
+        dem[-1, -1] = float("nan")
+    elif special == "all_nan":
+        dem[:] = float("nan")
+    elif special == "inf":
+        dem[h // 2, w // 2] = float("inf")
+    got = spatial.gaussian_nan(dem.to(cuda), pad, sigma).cpu().double().numpy()
+    x = np.pad(dem.double().numpy(), pad, mode="symmetric")
+    r = int(4.0 * sigma + 0.5)
+    g = np.exp(-0.5 / sigma ** 2 * np.arange(-r, r + 1) ** 2)
+    g /= g.sum()
+
+    def blur(a):
+        for ax in (0, 1):
+            p = np.pad(a, [(r, r) if k == ax else (0, 0) for k in (0, 1)], mode="edge")
+            a = sum(g[k] * np.take(p, range(k, k + a.shape[ax]), axis=ax)
+                    for k in range(2 * r + 1))
+        return a
+    bad = np.isnan(x)
+    with np.errstate(invalid="ignore"):
+        sw = blur((~bad).astype(np.float64))
+        want = np.where(sw > 0, blur(np.where(bad, 0.0, x)) / np.where(sw > 0, sw, 1.0), 0.0)
+    assert np.array_equal(np.isinf(got), np.isinf(want))
+    fin = np.isfinite(want)
+    assert np.all(np.abs(got[fin] - want[fin]) <= 4e-7 * np.abs(want[fin]))
