@@ -260,11 +260,13 @@ def _coarse_response(algorithm: str, coarse: torch.Tensor, r_c: int, p: dict) ->
 
 
 def _sample(resp: torch.Tensor, r0: int, c0: int, full_h: int, full_w: int,
-            win: torch.Tensor, out: torch.Tensor) -> None:
+            win: Optional[torch.Tensor], out: torch.Tensor) -> None:
+    """win: the window pixels whose NaN the sample takes over (None: it has none)."""
     N.check(N.lib().fsg_sample_coarse(resp.data_ptr(), resp.stride(0), resp.shape[0],
-                                      resp.shape[1], r0, c0, full_h, full_w, win.data_ptr(),
-                                      win.stride(0), out.data_ptr(), out.stride(0),
-                                      out.shape[0], out.shape[1], _s()))
+                                      resp.shape[1], r0, c0, full_h, full_w,
+                                      win.data_ptr() if win is not None else None,
+                                      win.stride(0) if win is not None else 0, out.data_ptr(),
+                                      out.stride(0), out.shape[0], out.shape[1], _s()))
 
 
 def field_radii(algorithm: str, p: dict, direct: bool = False):
@@ -335,7 +337,7 @@ def run(algorithm: str, win: torch.Tensor, reg: N.fsg_region, out_descs, p: dict
     fields: List[torch.Tensor] = []
     for r in [float(v) for v in radii]:
         field = torch.empty((reg.h, reg.w), dtype=torch.float32, device=win.device)
-        wsub = win[reg.r0:reg.r0 + reg.h, reg.c0:reg.c0 + reg.w]
+        wsub = None if nan_free else win[reg.r0:reg.r0 + reg.h, reg.c0:reg.c0 + reg.w]
         if direct:
             sm, may_nan = smooth_for_radius(win, 0, r, px, algorithm)
             _local(algorithm, sm, reg, field, base, nan_free=nan_free or not may_nan)

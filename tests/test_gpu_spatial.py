@@ -312,3 +312,69 @@ def test_gaussian_band_products_against_float64(cuda, h, w, pad, sigma, special)
     assert np.array_equal(np.isinf(got), np.isinf(want))
     fin = np.isfinite(want)
     assert np.all(np.abs(got[fin] - want[fin]) <= 4e-7 * np.abs(want[fin]))
+
+
+@pytest.mark.parametrize("h,w,hs,ws", [(1, 1, 1, 1), (17, 255, 5, 64), (64, 257, 16, 65),
+                                       (145, 600, 10, 38), (33, 130, 33, 130)])
+@pytest.mark.parametrize("nan", [False, True])
+def test_strip_kernels_at_ragged_extents(cuda, h, w, hs, ws, nan):
+    """Upsampling, the overview sample and the symmetric pad over partial strips and walks,
+    sources with and without voids, against the oracle.  Both interpolate in float64, in
+    another order, and round once to float32 (the upsampling's quotient once more), so
+    they differ by at most one unit (two) in the last place of the largest value."""
+    from fujishadergpu_amd import spatial
+    src = _dem(max(hs, 8), max(ws, 8), 61)[:hs, :ws].contiguous()
+    if nan:
+        src[hs // 2, ws // 2] = float("nan")
+        src[0, -1] = float("nan")
+    ulp = float(np.spacing(np.nanmax(np.abs(src.numpy()))))
+    _cmp("upsample", spatial.upsample_to_shape(src.to(cuda), h, w),
+         ref.upsample_to_shape(src.numpy(), (h, w)), 2 * ulp)
+    if not nan:
+        win = _dem(max(h, 8), max(w, 8), 62)[:h, :w].contiguous()
+        win[h // 2, w // 3] = float("nan")
+        for z in (None, win.to(cuda)):
+            out = torch.empty((h, w), dtype=torch.float32, device=cuda)
+            spatial._sample(src.to(cuda), 3, 5, h + 9, w + 40, z, out)
+            want = ref.bilinear_sample_coarse(src.numpy(), 3, 3 + h, 5, 5 + w, h + 9, w + 40)
+            if z is not None:
+                want = np.where(np.isnan(win.numpy()), np.float32(np.nan), want)
+            _cmp("sample", out, want, ulp)
+    d = min(hs, ws)
+    assert np.array_equal(spatial.pad_symmetric(src.to(cuda), d).cpu().numpy(),
+                          np.pad(src.numpy(), d, mode="symmetric"), equal_nan=True)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "int16", "uint8"])
+@pytest.mark.parametrize("agg", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("h,w,off", [(1, 1, 0), (5, 257, 1), (9, 1024, 3)])
+def test_combine_at_ragged_extents_and_offsets(cuda, dtype, agg, h, w, off):
+    """Every combination rule and encoding, output columns starting at odd addresses."""
+    import ctypes as C
+
+    from fujishadergpu_amd import _native as N
+    from fujishadergpu_amd import ops
+    from fujishadergpu_amd.encoding import quantize_params
+    qp = quantize_params(0.0, 1.0, dtype) if dtype != "float32" else None
+    g = torch.Generator().manual_seed(3)
+    f = torch.rand((3, h, w), generator=g)
+    f[1, 0, 0] = float("nan")
+    wts = np.array([0.5, 0.3, 0.2], np.float32)
+    a = f.numpy()
+    with np.errstate(invalid="ignore"):
+        want = {N.AGG_WEIGHTED: (a[0] * wts[0] + a[1] * wts[1]) + a[2] * wts[2],
+                N.AGG_MEAN: ((a[0] + a[1]) + a[2]) / np.float32(3), N.AGG_SUM: (a[0] + a[1]) + a[2],
+                N.AGG_MAX: a.max(0), N.AGG_MIN: a.min(0)}
+    kind = [N.AGG_WEIGHTED, N.AGG_MEAN, N.AGG_SUM, N.AGG_MAX, N.AGG_MIN][agg]
+    fd = f.to(cuda)
+    big = torch.zeros((h, w + 8), dtype=ops._TORCH_DTYPE[dtype], device=cuda)
+    out = ops.output(big[:, off:off + w], qp=qp)
+    ptrs = (C.c_void_p * 3)(*[fd[k].data_ptr() for k in range(3)])
+    N.check(N.lib().fsg_combine_fields(ptrs, 3, w, (C.c_float * 3)(*wts), kind, h, w,
+                                       C.byref(out), torch.cuda.current_stream().cuda_stream))
+    exp = want[kind]
+    if qp is not None:
+        exp = ref.quantize(exp, qp["a_coef"], qp["b_coef"], qp["dn_min"], qp["dn_max"], dtype)
+    got = big.cpu().numpy()
+    assert np.array_equal(got[:, off:off + w], exp, equal_nan=dtype == "float32")
+    assert not got[:, :off].any() and not got[:, off + w:].any()
