@@ -138,6 +138,30 @@ def openness_table(num_directions, max_distance, pixel_size=1.0, pixel_scale_x=N
     return table
 
 
+def openness_samples(num_directions, max_distance, pixel_size=1.0, pixel_scale_x=None,
+                     pixel_scale_y=None) -> np.ndarray:
+    """openness_table's entries as the (directions, distances) array of
+    fsg_ray_sample records that the kernels' entry points read."""
+    angles = np.linspace(0, 2 * np.pi, int(num_directions), endpoint=False)
+    dist = np.unique((np.linspace(0.1, 1.0, 10) * max_distance).astype(int))
+    dist = dist[dist > 0].astype(np.float64)
+    sx, sy = ray_steps(pixel_size, pixel_scale_x, pixel_scale_y)
+    return ops.ray_samples(np.rint(dist * np.cos(angles)[:, None]),
+                           np.rint(dist * np.sin(angles)[:, None]), sx, sy, ops.RAY_SAMPLE)
+
+
+def ao_samples(num_samples, radius, pixel_size=1.0, pixel_scale_x=None,
+               pixel_scale_y=None) -> np.ndarray:
+    """ao_table's entries as the array of fsg_ao_sample records."""
+    angles = np.linspace(0, 2 * np.pi, int(num_samples), endpoint=False)
+    rf = np.array([0.25, 0.5, 0.75, 1.0])[:, None]
+    sx, sy = ray_steps(pixel_size, pixel_scale_x, pixel_scale_y)
+    out = ops.ray_samples(np.round(radius * rf * np.cos(angles)),
+                          np.round(radius * rf * np.sin(angles)), sx, sy, ops.AO_SAMPLE)
+    out["dist_factor"] = 1.0 - (rf * 0.3)
+    return out.reshape(-1)
+
+
 def ao_table(num_samples, radius, pixel_size=1.0, pixel_scale_x=None, pixel_scale_y=None):
     """Ring table of compute_ambient_occlusion_block (_impl_ambient_occlusion.py:54-81)."""
     angles = np.linspace(0, 2 * np.pi, int(num_samples), endpoint=False)
@@ -431,9 +455,9 @@ class OpennessAlgorithm(NativeTileAlgorithm):
         if self.is_spatial(p):
             _run_spatial("openness", win, reg, out, p, post=post)
             return
-        table = openness_table(p.get("num_directions", 16), p.get("max_distance", 50),
-                               p.get("pixel_size", 1.0), p.get("pixel_scale_x"),
-                               p.get("pixel_scale_y"))
+        table = openness_samples(p.get("num_directions", 16), p.get("max_distance", 50),
+                                 p.get("pixel_size", 1.0), p.get("pixel_scale_x"),
+                                 p.get("pixel_scale_y"))
         for o in out.descriptors(*post):
             ops.openness(win, reg, table=table,
                          openness_type=p.get("openness_type", "positive"), out=o)
@@ -456,8 +480,8 @@ class AmbientOcclusionAlgorithm(NativeTileAlgorithm):
             _run_spatial("ambient_occlusion", win, reg, out, p, post=post)
             return
         radius = p.get("radius", 10.0)
-        table = ao_table(p.get("num_samples", 16), radius, p.get("pixel_size", 1.0),
-                         p.get("pixel_scale_x"), p.get("pixel_scale_y"))
+        table = ao_samples(p.get("num_samples", 16), radius, p.get("pixel_size", 1.0),
+                           p.get("pixel_scale_x"), p.get("pixel_scale_y"))
         for o in out.descriptors(*post):
             ops.ambient_occlusion(win, reg, table=table, intensity=p.get("intensity", 1.0),
                                   pad_d=max(1, int(round(float(radius)))), out=o)

@@ -144,9 +144,33 @@ def curvature(win_t, reg, *, step_x: float, step_y: float, curvature_type: str,
 
 # ------------------------------------------------------------------ rays
 
+# the records of fsg_ray_sample and fsg_ao_sample
+RAY_SAMPLE = np.dtype([("dx", "<i4"), ("dy", "<i4"), ("skip", "<i4"), ("pad0", "<i4"),
+                       ("phys", "<f8")])
+AO_SAMPLE = np.dtype(RAY_SAMPLE.descr + [("dist_factor", "<f8")])
+
+
+def ray_samples(ox: np.ndarray, oy: np.ndarray, sx: float, sy: float,
+                dtype: np.dtype) -> np.ndarray:
+    """Sample records at whole pixel offsets (ox, oy): the physical distance for
+    pixel steps (sx, sy), at least 1e-9; the pixel itself is skipped."""
+    out = np.zeros(ox.shape, dtype=dtype)
+    out["dx"], out["dy"] = ox, oy
+    out["skip"] = (ox == 0) & (oy == 0)
+    out["phys"] = np.maximum(np.hypot(ox * sx, oy * sy), 1e-9)
+    return out
+
+
 def openness_params(table, openness_type: str, raw_degrees: bool = False):
-    """(params, keep-alive array) for a ray table: list over directions of
-    lists over distances of (ox, oy, phys)|None."""
+    """(params, keep-alive array) for a ray table: a (directions, distances)
+    RAY_SAMPLE array, or a list over directions of lists over distances of
+    (ox, oy, phys)|None."""
+    if isinstance(table, np.ndarray):
+        arr = np.ascontiguousarray(table, dtype=RAY_SAMPLE)
+        return N.fsg_openness_params(
+            0 if openness_type == "positive" else 1, arr.shape[0], arr.shape[1],
+            1 if raw_degrees else 0,
+            C.cast(arr.ctypes.data, C.POINTER(N.fsg_ray_sample))), arr
     n_dirs = len(table)
     n_dist = max((len(r) for r in table), default=0)
     arr = (N.fsg_ray_sample * max(1, n_dirs * n_dist))()
@@ -245,16 +269,17 @@ def openness_judge(win_t, approx: torch.Tensor, *, tile_h: int, tile_w: int, sam
 
 def ambient_occlusion(win_t, reg, *, table, intensity: float, pad_d: int,
                       out: N.fsg_output) -> None:
-    """table: list of (dx, dy, phys, dist_factor)|None in reference order."""
-    arr = (N.fsg_ao_sample * max(1, len(table)))()
-    for i, entry in enumerate(table):
-        if entry is None:
-            arr[i].skip = 1
-        else:
-            arr[i].dx, arr[i].dy = int(entry[0]), int(entry[1])
-            arr[i].phys, arr[i].dist_factor = float(entry[2]), float(entry[3])
-    p = N.fsg_ao_params(len(table), int(pad_d), float(intensity),
-                        C.cast(arr, C.POINTER(N.fsg_ao_sample)))
+    """table: an AO_SAMPLE array, or a list of (dx, dy, phys, dist_factor)|None, in
+    reference order."""
+    if isinstance(table, np.ndarray):
+        arr = np.ascontiguousarray(table, dtype=AO_SAMPLE)
+    else:
+        arr = np.zeros(len(table), dtype=AO_SAMPLE)
+        for i, entry in enumerate(table):
+            arr[i] = (0, 0, 1, 0, 0.0, 0.0) if entry is None else \
+                (int(entry[0]), int(entry[1]), 0, 0, float(entry[2]), float(entry[3]))
+    p = N.fsg_ao_params(len(arr), int(pad_d), float(intensity),
+                        C.cast(arr.ctypes.data, C.POINTER(N.fsg_ao_sample)))
     w = window(win_t)
     L = _lib()
     nbytes = L.fsg_ambient_occlusion_workspace_size(C.byref(w), C.byref(reg))

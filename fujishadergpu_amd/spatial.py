@@ -203,16 +203,16 @@ def _ray_local(algorithm: str, src: torch.Tensor, reg: N.fsg_region, out: torch.
                r: float, p: dict) -> None:
     """compute_openness_vectorized / compute_ambient_occlusion_block of src at
     radius r (max_distance / radius), region reg into out (no display stretch)."""
-    from .algorithms import ao_table, openness_table
+    from .algorithms import ao_samples, openness_samples
     px = p.get("pixel_size", 1.0)
     psx, psy = p.get("pixel_scale_x"), p.get("pixel_scale_y")
     o = ops.output(out)
     if algorithm == "openness":
-        table = openness_table(p.get("num_directions", 16), r, px, psx, psy)
+        table = openness_samples(p.get("num_directions", 16), r, px, psx, psy)
         ops.openness(src, reg, table=table, openness_type=p.get("openness_type", "positive"),
                      out=o)
     else:
-        table = ao_table(p.get("num_samples", 16), r, px, psx, psy)
+        table = ao_samples(p.get("num_samples", 16), r, px, psx, psy)
         ops.ambient_occlusion(src, reg, table=table, intensity=p.get("intensity", 1.0),
                               pad_d=max(1, int(round(float(r)))), out=o)
 

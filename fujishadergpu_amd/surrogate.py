@@ -41,7 +41,7 @@ import torch
 
 from . import _native as N
 from . import ops, synth
-from .algorithms import openness_table
+from .algorithms import openness_samples
 
 WIDTHS = (8, 32, 32, 32, 32, 32, 2)      # input channels (4 real + 4 zero) ... output
 GRID = 8                                   # network grid factor
@@ -235,7 +235,7 @@ def _up(src: torch.Tensor, factor: int, h: int, w: int, add=None) -> torch.Tenso
 def exact_openness(win: torch.Tensor, reg, radius: int, n_dirs: int, pixel_size: float,
                    out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Exact openness angle (degrees) of the region (the reference's sparse rays)."""
-    tab = openness_table(n_dirs, radius, pixel_size, None, None)
+    tab = openness_samples(n_dirs, radius, pixel_size, None, None)
     if out is None:
         out = torch.empty((reg.h, reg.w), dtype=torch.float32, device=win.device)
     ops.openness(win, reg, table=tab, openness_type="positive", out=ops.output(out),
@@ -482,7 +482,7 @@ def judge(win: torch.Tensor, approx: torch.Tensor, radius: int, n_dirs: int, pix
     coalesce -- and every tile whose mean absolute error on them exceeds the
     threshold recomputed exactly in place."""
     H, W = win.shape
-    tab = openness_table(n_dirs, radius, pixel_size, None, None)
+    tab = openness_samples(n_dirs, radius, pixel_size, None, None)
     tiles = [(y0, x0, min(tile, H - y0), min(tile, W - x0))
              for y0 in range(0, H, tile) for x0 in range(0, W, tile)]
     seg_len = min(SEG, min(tw for _, _, _, tw in tiles))

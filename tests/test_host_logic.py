@@ -240,3 +240,25 @@ def test_raster_job_refuses_the_multi_radius_hillshade():
     assert len(HillshadeAlgorithm._direct_radii(P.params)) > 1
     P1 = plan(torch.zeros(2600, 3100), "hillshade", tile_size=1024, pixel_size=10.0, radii=[1])
     assert HillshadeAlgorithm._direct_radii(P1.params) == [1.0]
+
+
+@pytest.mark.parametrize("n,dist,px,sx,sy", [(16, 50, 1.0, None, None), (8, 64, 10.0, 10.0, -10.0),
+                                             (7, 3, 5.0, 23.4, 30.9), (1, 1024, 2.0, None, -2.0),
+                                             (16, 2.0, 1e-12, None, None)])
+def test_ray_sample_arrays_equal_the_tables(n, dist, px, sx, sy):
+    """The record arrays that the entry points read hold the tables' values bit for bit."""
+    from fujishadergpu_amd import ops
+    from fujishadergpu_amd.algorithms import (ao_samples, ao_table, openness_samples,
+                                              openness_table)
+    table = openness_table(n, dist, px, sx, sy)
+    got = openness_samples(n, dist, px, sx, sy)
+    want = ops.openness_params(table, "positive")[1]
+    assert got.shape == (len(table), len(table[0]))
+    for g, w in zip(got.reshape(-1), want):
+        assert int(g["skip"]) == w.skip
+        if not w.skip:
+            assert (int(g["dx"]), int(g["dy"]), float(g["phys"])) == (w.dx, w.dy, w.phys)
+    for g, w in zip(ao_samples(n, float(dist), px, sx, sy), ao_table(n, float(dist), px, sx, sy)):
+        assert bool(g["skip"]) == (w is None)
+        if w is not None:
+            assert (int(g["dx"]), int(g["dy"]), float(g["phys"]), float(g["dist_factor"])) == w
