@@ -25,6 +25,7 @@
 #include <cmath>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "usm.hpp"
@@ -242,54 +243,87 @@ __device__ __forceinline__ double vf_w(const VFWeights& V, int d) {
   return V.by_value ? V.g[d] : exp(-0.5 / V.sigma2 * (double)(d * d)) * V.inv_sum;
 }
 
-__global__ void k_voidfill_pass(const float* __restrict__ a, const float* __restrict__ b,
-                                float* __restrict__ oa, float* __restrict__ ob, int h, int w,
-                                VFWeights V, int axis, const int* __restrict__ nan_flag) {
+// Only void cells change, and few rows hold one nearby: seg[r][s] tells whether
+// cells 64 s .. 64 s + 63 of row r hold a void, pass 0 computes the segments
+// within the filter's reach of one, and pass 1 the void cells themselves, which
+// it fills in place.  A wave takes one row segment at a time (over every cell
+// the two passes took 28 us each on the coarse grids of a 9001 x 7003 job with
+// 1 % NoData; now 14 and 12).
+__global__ void __launch_bounds__(256)
+k_voidfill_seg(const float* __restrict__ a, int h, int w, int nseg,
+               unsigned char* __restrict__ seg, const int* __restrict__ nan_flag) {
   if (*nan_flag == 0) return;
-  const int rad = V.rad;
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < (int64_t)h * w;
-       e += (int64_t)gridDim.x * blockDim.x) {
-  const int r = (int)(e / w), c = (int)(e - (int64_t)r * w);
-  double sv, sw;
-  if (axis == 0) {
-    // a = coarse (NaN -> value 0, weight 0)
+  const int lane = threadIdx.x & 63;
+  for (int e = blockIdx.x * 4 + (threadIdx.x >> 6); e < h * nseg; e += gridDim.x * 4) {
+    const int r = e / nseg, c = (e - r * nseg) * 64 + lane;
+    const bool v = c < w && isnan(a[(int64_t)r * w + c]);
+    const bool any = __builtin_amdgcn_ballot_w64(v) != 0;
+    if (lane == 0) seg[e] = any ? 1 : 0;
+  }
+}
+
+// Pass 0, axis 0: (where(nan, 0, x), valid) -> (tv, tw).
+__global__ void __launch_bounds__(256)
+k_voidfill_cols(const float* __restrict__ a, float* __restrict__ tv, float* __restrict__ tw, int h,
+                int w, int nseg, const unsigned char* __restrict__ seg, VFWeights V,
+                const int* __restrict__ nan_flag) {
+  if (*nan_flag == 0) return;
+  const int lane = threadIdx.x & 63;
+  const int k = (V.rad + 63) / 64;   // segments either side within reach
+  for (int e = blockIdx.x * 4 + (threadIdx.x >> 6); e < h * nseg; e += gridDim.x * 4) {
+    const int r = e / nseg, s = e - r * nseg;
+    bool near = false;
+    for (int q = max(s - k, 0) + lane; q <= min(s + k, nseg - 1); q += 64)
+      near |= seg[r * nseg + q] != 0;
+    if (__builtin_amdgcn_ballot_w64(near) == 0) continue;
+    const int c = s * 64 + lane;
+    if (c >= w) continue;
     const float x0 = a[(int64_t)r * w + c];
-    sv = (isnan(x0) ? 0.0 : (double)x0) * vf_w(V, 0);
-    sw = (isnan(x0) ? 0.0 : 1.0) * vf_w(V, 0);
-    for (int d = rad; d >= 1; d--) {
+    double sv = (isnan(x0) ? 0.0 : (double)x0) * vf_w(V, 0);
+    double sw = (isnan(x0) ? 0.0 : 1.0) * vf_w(V, 0);
+#pragma unroll 4
+    for (int d = V.rad; d >= 1; d--) {
       const float xa = a[(int64_t)clampi(r - d, h) * w + c];
       const float xb = a[(int64_t)clampi(r + d, h) * w + c];
-      sv += ((isnan(xa) ? 0.0 : (double)xa) + (isnan(xb) ? 0.0 : (double)xb)) * vf_w(V, d);
-      sw += ((isnan(xa) ? 0.0 : 1.0) + (isnan(xb) ? 0.0 : 1.0)) * vf_w(V, d);
+      const double g = vf_w(V, d);
+      sv += ((isnan(xa) ? 0.0 : (double)xa) + (isnan(xb) ? 0.0 : (double)xb)) * g;
+      sw += ((isnan(xa) ? 0.0 : 1.0) + (isnan(xb) ? 0.0 : 1.0)) * g;
     }
-  } else {
-    const int64_t row = (int64_t)r * w;
-    sv = (double)a[row + c] * vf_w(V, 0);
-    sw = (double)b[row + c] * vf_w(V, 0);
-    for (int d = rad; d >= 1; d--) {
-      sv += ((double)a[row + clampi(c - d, w)] + (double)a[row + clampi(c + d, w)]) * vf_w(V, d);
-      sw += ((double)b[row + clampi(c - d, w)] + (double)b[row + clampi(c + d, w)]) * vf_w(V, d);
-    }
+    tv[(int64_t)r * w + c] = (float)sv;
+    tw[(int64_t)r * w + c] = (float)sw;
   }
-  oa[(int64_t)r * w + c] = (float)sv;
-  ob[(int64_t)r * w + c] = (float)sw;
+}
+
+// Pass 1, axis 1, and coarse = where(isnan & sw > 0.5, sv / max(sw, 1e-6), coarse).
+__global__ void __launch_bounds__(256)
+k_voidfill_rows(float* __restrict__ coarse, const float* __restrict__ tv,
+                const float* __restrict__ tw, int h, int w, int nseg,
+                const unsigned char* __restrict__ seg, VFWeights V,
+                const int* __restrict__ nan_flag) {
+  if (*nan_flag == 0) return;
+  const int lane = threadIdx.x & 63;
+  for (int e = blockIdx.x * 4 + (threadIdx.x >> 6); e < h * nseg; e += gridDim.x * 4) {
+    if (!seg[e]) continue;
+    const int r = e / nseg, c = (e - r * nseg) * 64 + lane;
+    const int64_t row = (int64_t)r * w;
+    if (c >= w || !isnan(coarse[row + c])) continue;
+    double sv = (double)tv[row + c] * vf_w(V, 0);
+    double sw = (double)tw[row + c] * vf_w(V, 0);
+#pragma unroll 4
+    for (int d = V.rad; d >= 1; d--) {
+      const int ca = clampi(c - d, w), cb = clampi(c + d, w);
+      const double g = vf_w(V, d);
+      sv += ((double)tv[row + ca] + (double)tv[row + cb]) * g;
+      sw += ((double)tw[row + ca] + (double)tw[row + cb]) * g;
+    }
+    const float fv = (float)sv, fw = (float)sw;
+    if (fw > 0.5f) coarse[row + c] = fv / fmaxf(fw, 1e-6f);
   }
 }
 
 __global__ void k_zero_int(int* __restrict__ p, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0;
-}
-
-// coarse = where(isnan & sw > 0.5, sv / max(sw, 1e-6), coarse)
-__global__ void k_voidfill_apply(float* __restrict__ coarse, const float* __restrict__ sv,
-                                 const float* __restrict__ sw, int n,
-                                 const int* __restrict__ nan_flag) {
-  if (*nan_flag == 0) return;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const float x = coarse[i];
-    if (isnan(x) && sw[i] > 0.5f) coarse[i] = sv[i] / fmaxf(sw[i], 1e-6f);
-  }
 }
 
 // NaN-aware box mean on a small grid as two transposing axis-0 passes.  A
@@ -299,7 +333,7 @@ __global__ void k_voidfill_apply(float* __restrict__ coarse, const float* __rest
 //   pass 0: x (h x w, NaN-aware)  -> tv^T, tw^T (w x h): float32 axis-0 means
 //   pass 1: tv^T, tw^T (w x h)    -> out (h x w): axis-1 means of those and
 //           where(sw > 0, sv / sw, 0)   (_nan_utils.py:34-47 structure)
-template <int PASS>
+template <int PASS, int BAND>
 __device__ __forceinline__ void box_t_block(const float* __restrict__ a,
                                             const float* __restrict__ b, int64_t lda, int h,
                                             int w, int r, double inv, float* __restrict__ oa,
@@ -307,8 +341,8 @@ __device__ __forceinline__ void box_t_block(const float* __restrict__ a,
                                             float (*ta)[65], float (*tb)[65]) {
   const int lane = threadIdx.x;
   const int c = bx * 64 + lane;  // column of the (h x w) input
-  const int y0 = by * 64;
-  const int y1 = min(y0 + 64, h);
+  const int y0 = by * BAND;
+  const int y1 = min(y0 + BAND, h);
   if (c < w) {
     const float* pa = a + c;
     const float* pb = PASS ? b + c : nullptr;
@@ -373,23 +407,24 @@ __device__ __forceinline__ void box_t_block(const float* __restrict__ a,
   __syncthreads();
   // transposed write: output row = input column, output column = input row
   const int ncol = min(64, w - bx * 64);
-  for (int cc = 0; cc < ncol; cc++) {
-    const int y = y0 + lane;
-    if (y < y1) {
+  for (int c0 = 0; c0 < ncol; c0 += 64 / BAND) {
+    const int cc = c0 + lane / BAND, k = lane % BAND;
+    const int y = y0 + k;
+    if (y < y1 && cc < ncol) {
       const int64_t o = (int64_t)(bx * 64 + cc) * ldo + y;
-      oa[o] = ta[lane][cc];
-      if (PASS == 0) ob[o] = tb[lane][cc];
+      oa[o] = ta[k][cc];
+      if (PASS == 0) ob[o] = tb[k][cc];
     }
   }
 }
 
-template <int PASS>
+template <int PASS, int BAND>
 __global__ void __launch_bounds__(64)
 k_box_t(const float* __restrict__ a, const float* __restrict__ b, int64_t lda, int h, int w,
         int r, double inv, float* __restrict__ oa, float* __restrict__ ob, int64_t ldo) {
-  __shared__ float ta[64][65];
-  __shared__ float tb[64][65];
-  box_t_block<PASS>(a, b, lda, h, w, r, inv, oa, ob, ldo, blockIdx.x, blockIdx.y, ta, tb);
+  __shared__ float ta[BAND][65];
+  __shared__ float tb[BAND][65];
+  box_t_block<PASS, BAND>(a, b, lda, h, w, r, inv, oa, ob, ldo, blockIdx.x, blockIdx.y, ta, tb);
 }
 
 // Box passes of several independent grids in one launch (see k_decimate_batch).
@@ -401,7 +436,7 @@ k_box_t_batch(const BoxJob* __restrict__ jobs, const int* __restrict__ pre, int 
   const int j = batch_job_of(pre, n, blockIdx.x);
   const BoxJob J = jobs[j];
   const int local = blockIdx.x - pre[j];
-  box_t_block<PASS>(J.a, J.b, J.lda, J.h, J.w, J.r, J.inv, J.oa, J.ob, J.ldo, local % J.nbx,
+  box_t_block<PASS, 64>(J.a, J.b, J.lda, J.h, J.w, J.r, J.inv, J.oa, J.ob, J.ldo, local % J.nbx,
                     local / J.nbx, ta, tb);
 }
 
@@ -1254,20 +1289,31 @@ static int coarse_mean(const float* x, int64_t ldx, int h, int w, int r, float* 
     return FSG_OK;
   }
   const double inv = 1.0 / (double)(2 * r + 1);
-  // pass 0: (h x w) -> transposed (w x h) axis-0 means
-  hipLaunchKernelGGL(k_box_t<0>, dim3((w + 63) / 64, (h + 63) / 64), dim3(64), 0, s, x,
-                     nullptr, ldx, h, w, r, inv, tv, tw, (int64_t)h);
-  FSG_CHECK_LAUNCH("k_box_t");
-  // pass 1: axis 0 of the transposed grid (= axis 1), transposed back
-  hipLaunchKernelGGL(k_box_t<1>, dim3((h + 63) / 64, (w + 63) / 64), dim3(64), 0, s, tv, tw,
-                     (int64_t)h, w, h, r, inv, out, nullptr, ldo);
+  // pass 0: (h x w) -> transposed (w x h) axis-0 means; pass 1: axis 0 of the
+  // transposed grid (= axis 1), transposed back.  A block is one wave whose chain
+  // of load batches lasts as long as its band; a grid of few blocks takes bands of
+  // 16 rows instead of 64 while the 2 r + 1 start-up rows stay below 81 (1104^2
+  // grids, r = 32: 36 and 33 us a pass with 64 rows, 21 and 20 with 16).
+  const bool flat = r <= 40 && (int64_t)((w + 63) / 64) * ((h + 63) / 64) < 1024;
+  const auto launch = [&](auto band) {
+    constexpr int BAND = decltype(band)::value;
+    hipLaunchKernelGGL((k_box_t<0, BAND>), dim3((w + 63) / 64, (h + BAND - 1) / BAND), dim3(64),
+                       0, s, x, nullptr, ldx, h, w, r, inv, tv, tw, (int64_t)h);
+    hipLaunchKernelGGL((k_box_t<1, BAND>), dim3((h + 63) / 64, (w + BAND - 1) / BAND), dim3(64),
+                       0, s, tv, tw, (int64_t)h, w, h, r, inv, out, nullptr, ldo);
+  };
+  if (flat)
+    launch(std::integral_constant<int, 16>{});
+  else
+    launch(std::integral_constant<int, 64>{});
+  count_launch();
   FSG_CHECK_LAUNCH("k_box_t");
   return FSG_OK;
 }
 
 // Decimated grid with the enclosed-void fill (_nan_utils.py:604-668).
 static int decimate(const fsg_window* win, int ds, float* grid, int hc, int wc, int* flag,
-                    float* t0, float* t1, float* t2, float* t3, bool nan_free, hipStream_t s) {
+                    float* t0, float* t1, float* t2, bool nan_free, hipStream_t s) {
   if (ds > 16 || (ds & (ds - 1)) != 0)
     return fail(FSG_E_UNSUPPORTED, "fsg_topousm: downsample factor must be a power of two <= 16");
   hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(64), 0, s, flag, 1);
@@ -1305,14 +1351,15 @@ static int decimate(const fsg_window* win, int ds, float* grid, int hc, int wc, 
       V.inv_sum = 1.0 / np_pairwise_sum(phi.data(), 2 * rad + 1);
     }
   }
-  const int n = hc * wc;
-  dim3 blk(256), grd(std::min(1024, (n + 255) / 256));
-  hipLaunchKernelGGL(k_voidfill_pass, grd, blk, 0, s, grid, grid, t0, t1, hc, wc, V, 0, flag);
-  FSG_CHECK_LAUNCH("k_voidfill_pass");
-  hipLaunchKernelGGL(k_voidfill_pass, grd, blk, 0, s, t0, t1, t2, t3, hc, wc, V, 1, flag);
-  FSG_CHECK_LAUNCH("k_voidfill_pass");
-  hipLaunchKernelGGL(k_voidfill_apply, grd, blk, 0, s, grid, t2, t3, n, flag);
-  FSG_CHECK_LAUNCH("k_voidfill_apply");
+  const int nseg = (wc + 63) / 64;
+  unsigned char* seg = (unsigned char*)t2;
+  const dim3 blk(256), grd(std::min(4096, (hc * nseg + 3) / 4));
+  hipLaunchKernelGGL(k_voidfill_seg, grd, blk, 0, s, grid, hc, wc, nseg, seg, flag);
+  FSG_CHECK_LAUNCH("k_voidfill_seg");
+  hipLaunchKernelGGL(k_voidfill_cols, grd, blk, 0, s, grid, t0, t1, hc, wc, nseg, seg, V, flag);
+  FSG_CHECK_LAUNCH("k_voidfill_cols");
+  hipLaunchKernelGGL(k_voidfill_rows, grd, blk, 0, s, grid, t0, t1, hc, wc, nseg, seg, V, flag);
+  FSG_CHECK_LAUNCH("k_voidfill_rows");
   return FSG_OK;
 }
 
@@ -1396,7 +1443,7 @@ int fsg::usm_prepare(const fsg_window* win, const fsg_region* reg, const fsg_top
   for (int k = 0; k < 4; k++) tmp[k] = (float*)(ws + P.tmp_off[k]);
   for (int j = 0; j < P.n_ds && launch_prep; j++) {
     rc = decimate(win, P.ds_val[j], (float*)(ws + P.grid_off[j]), P.hc[j], P.wc[j], flags + j,
-                  tmp[0], tmp[1], tmp[2], tmp[3], p->nan_hint == 0, s);
+                  tmp[0], tmp[1], tmp[2], p->nan_hint == 0, s);
     if (rc) return rc;
   }
   // Fast path when the terms run [distinct box radii in slot order][decimated
@@ -1703,7 +1750,7 @@ extern "C" int fsg_downsample_nan_aware(const fsg_window* src, int32_t factor, f
   float* t[4];
   for (int k = 0; k < 4; k++) t[k] = (float*)(ws + k * g);
   int* flag = (int*)(ws + 4 * g);
-  return decimate(src, factor, out, hc, wc, flag, t[0], t[1], t[2], t[3], false,
+  return decimate(src, factor, out, hc, wc, flag, t[0], t[1], t[2], false,
                   as_stream(stream));
 }
 
@@ -1816,7 +1863,7 @@ extern "C" int fsg_topousm_coarse_means(const fsg_window* win, int32_t ds, int32
     grid = const_cast<float*>(win->data);
     ldg = win->ld;
   } else {
-    rc = decimate(win, ds, grid, hc, wc, flag, tmp[0], tmp[1], tmp[2], tmp[3], false, s);
+    rc = decimate(win, ds, grid, hc, wc, flag, tmp[0], tmp[1], tmp[2], false, s);
     if (rc) return rc;
   }
   for (int i = 0; i < n_radii; i++) {

@@ -701,3 +701,37 @@ def test_ambient_occlusion_tiles_match_the_oracle(cuda, h, w, samples, radius, p
                                  pixel_size=px)
     assert np.array_equal(np.isnan(got), np.isnan(want))
     assert np.nanmax(np.abs(got - want)) < 1e-5
+
+
+@pytest.mark.parametrize("h,w,f", [(2, 2, 2), (130, 126, 2), (260, 520, 4), (90, 2600, 2),
+                                   (2210, 2200, 2)])
+def test_enclosed_void_fill_at_segment_edges(cuda, h, w, f):
+    """The decimated grid's void fill, which computes only the row segments near a void,
+    against the oracle: voids across segments, at the edges, a reach beyond a segment
+    (the widest grid), and a grid that is all void but one cell."""
+    from fujishadergpu_amd import spatial, synth
+    dem = synth.fbm(max(h, 8), max(w, 8), 0.7, 800.0, seed=9)[:h, :w].contiguous()
+    holes = [(h // 2, w // 2 - 9, 12, 40), (0, 0, f, f), (h - f, w - 3 * f, f, 3 * f),
+             (h // 4, min(w - f, 126), f, f)]
+    for y, x, dy, dx in holes:
+        dem[y:y + dy, max(x, 0):x + dx] = float("nan")
+    for d in (dem, torch.where(torch.arange(h * w).view(h, w) >= f, float("nan"), dem)):
+        got = spatial.downsample_nan_aware(d.to(cuda), f).cpu().numpy()
+        want = ref.downsample_nan_aware(d.numpy(), f)
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        ok = ~np.isnan(want)
+        # a few float32 roundings of sums of heights below 800
+        assert not ok.any() or np.abs(got[ok] - want[ok]).max() <= 3e-4
+
+
+@pytest.mark.parametrize("h,w,radii", [(17, 16, [2]), (130, 67, [2, 40]), (65, 300, [41, 8]),
+                                       (2100, 2200, [32])])
+def test_nan_aware_box_bands_match_the_oracle(cuda, h, w, radii):
+    """Box means of grids on both sides of the flat-band rule (radius 40, 1024 blocks)."""
+    from fujishadergpu_amd import ops, synth
+    dem = synth.fbm(h, w, 0.7, 800.0, seed=12)
+    dem[h // 3:h // 3 + 9, w // 2:w // 2 + 5] = float("nan")
+    got = ops.topousm_coarse_means(dem.to(cuda), 1, radii).cpu().numpy()
+    for g, r in zip(got, radii):
+        want, _ = ref.handle_nan_with_uniform(dem.numpy(), size=2 * r + 1, mode="reflect")
+        assert np.abs(g - want).max() <= 3e-4
