@@ -986,23 +986,6 @@ static int launch_fast(const UsmArgs& A, int n_tiles, hipStream_t s) {
 // 0: the wavefront kernel wherever it applies; 1: the workgroup kernels only
 static std::atomic<int> g_usm_variant{0};
 
-// One launch: the blocks whose rows and columns all lie inside the window
-// (no reflection) take the FAST = true code, the others the reflecting loads.
-template <int NR, int NS, int KR>
-__device__ __forceinline__ void wave_tile(const WaveArgs& A, int tile, double* P, double* Hc) {
-  const int x0 = (tile % A.n_strips) * A.SW;
-  const int y0 = (tile / A.n_strips) * A.SH;
-  const int rows = min(A.SH, A.rh - y0);
-  const int cs = A.c0 + x0 - A.R;
-  const int wy0 = A.r0 + y0;
-  const bool fast = cs >= 0 && cs + WAVE_NC <= A.W && wy0 - A.R - 1 >= 0 &&
-                    wy0 + rows - 1 + A.R <= A.H - 1;
-  if (fast)
-    usm_wave_block<NR, NS, true, KR>(A, tile, P, Hc);
-  else
-    usm_wave_block<NR, NS, false, KR>(A, tile, P, Hc);
-}
-
 // Block b takes tile (b & 7) * per_xcd + (b >> 3): consecutive tiles of a
 // strip (vertical neighbours, sharing halo rows) land on one XCD and its L2.
 template <int NR, int NS, int KR>
@@ -1012,7 +995,8 @@ __global__ void __launch_bounds__(64) k_usm_wave(WaveArgs A) {
   const int b = blockIdx.x;
   const int tile = (b & 7) * A.per_xcd + (b >> 3);
   if (tile >= A.n_blocks) return;
-  wave_tile<NR, NS, KR>(A, tile, P, Hc);
+  const bool bad = wave_tile<NR, NS, KR, WAVE_CHECK>(A, tile, P, Hc);
+  if (A.flags && threadIdx.x == 0) A.flags[tile] = bad ? 1 : 0;
 }
 
 // Many windows' wavefront main passes in one launch (fsg_batch): block b
@@ -1035,7 +1019,7 @@ __global__ void __launch_bounds__(64) k_usm_wave_batch(const WaveArgs* args, con
   const int local = b - desc(pre, lo);
   const int tile = (local & 7) * A.per_xcd + (local >> 3);
   if (tile >= A.n_blocks) return;
-  wave_tile<NR, NS, KR>(A, tile, P, Hc);
+  wave_tile<NR, NS, KR, WAVE_PLAIN>(A, tile, P, Hc);
 }
 
 // Bilinear row coefficients of every source at every region row (the same
@@ -1093,17 +1077,27 @@ static int launch_wave(WaveArgs A, hipStream_t s) {
   A.SH = wave_rows(A.rh, A.n_strips, wave_capacity<NR, NS, KR>());
   A.n_blocks = A.n_strips * ((A.rh + A.SH - 1) / A.SH);
   A.per_xcd = (A.n_blocks + 7) / 8;
-  TimedScope ts("k_usm_main", s);
-  hipLaunchKernelGGL((k_usm_wave<NR, NS, KR>), dim3(A.per_xcd * 8), dim3(64), 0, s, A);
-  FSG_CHECK_LAUNCH("k_usm_wave");
-  return FSG_OK;
+  {
+    TimedScope ts("k_usm_main", s);
+    hipLaunchKernelGGL((k_usm_wave<NR, NS, KR>), dim3(A.per_xcd * 8), dim3(64), 0, s, A);
+    FSG_CHECK_LAUNCH("k_usm_wave");
+  }
+  return A.flags ? launch_wave_nan(A, NR, NS, s) : FSG_OK;
 }
 
-// The wavefront kernel handles NaN-free windows in the fast term order with
-// 1..3 box radii up to 32 and at most 3 bilinear sources.
+// The wavefront kernel handles windows in the fast term order with 1..3 box
+// radii up to 32 and at most 3 bilinear sources; with NaN (nanaw) its blocks'
+// marks (at most one per strip and 8 rows: the sweeps' smallest block) must fit
+// what the tables of at most three sources leave of their area.
+static size_t wave_marks(const UsmArgs& A) {
+  const size_t strips = (A.rw + WAVE_NC - 2 * A.R - 1) / (WAVE_NC - 2 * A.R);
+  return strips * ((size_t)A.rh / 8 + 1);
+}
 static bool wave_eligible(const UsmArgs& A, bool nanaw) {
-  return g_usm_variant.load(std::memory_order_relaxed) != 1 && !nanaw && A.nr >= 1 &&
-         A.nr <= WAVE_MAX_NR && A.R <= WAVE_MAX_R && A.n_src <= WAVE_MAX_SRC;
+  return g_usm_variant.load(std::memory_order_relaxed) != 1 && A.nr >= 1 &&
+         A.nr <= WAVE_MAX_NR && A.R <= WAVE_MAX_R && A.n_src <= WAVE_MAX_SRC &&
+         (!nanaw || wave_marks(A) <= sizeof(int4) * ((size_t)MAX_SRC * (A.W.h + A.W.w) -
+                                                     (size_t)A.n_src * A.rh));
 }
 
 // The wavefront kernel's arguments for a fast-path call (coefficient tables
@@ -1154,10 +1148,11 @@ static int wave_args(const UsmArgs& U, int4* tab, WaveArgs& A, hipStream_t s) {
 
 // Builds the coefficient tables and launches the wavefront kernel for the
 // arguments of a fast-path call.
-static int dispatch_wave(const UsmArgs& U, int4* tab, hipStream_t s) {
+static int dispatch_wave(const UsmArgs& U, int4* tab, bool nanaw, hipStream_t s) {
   WaveArgs A;
   const int rc = wave_args(U, tab, A, s);
   if (rc) return rc;
+  if (nanaw) A.flags = (unsigned char*)(tab + (size_t)U.n_src * U.rh);
   if (U.nr == 3 && U.rad[0] == 2 && U.rad[1] == 8 && U.rad[2] == 32) {
     if (U.n_src == 0) return launch_wave<3, 0, 1>(A, s);
     if (U.n_src == 1) return launch_wave<3, 1, 1>(A, s);
@@ -1769,7 +1764,8 @@ extern "C" int fsg_topousm(const fsg_window* win, const fsg_region* reg,
   // knows the window holds no NaN) selects the cheaper plain-mean variant,
   // whose results are identical on NaN-free windows.
   if (fast && wave_eligible(A, p->nan_hint != 0))
-    return dispatch_wave(A, (int4*)((char*)workspace + plan_coarse(win, p).tab_off), s);
+    return dispatch_wave(A, (int4*)((char*)workspace + plan_coarse(win, p).tab_off),
+                         p->nan_hint != 0, s);
   if (fast) return dispatch_fast(A, /*nanaw=*/p->nan_hint != 0, n_blocks, s);
   return dispatch_usm(A, /*nanaw=*/p->nan_hint != 0, n_blocks, s);
 }

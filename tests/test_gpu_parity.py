@@ -663,6 +663,73 @@ def test_wave_kernel_equals_the_workgroup_kernel(cuda, radii, weights, px, shape
     print("radii", radii, "max |d| vs oracle", mx, flush=True)
 
 
+@pytest.mark.parametrize("radii,px,shape,reg,field,holes,variant", [
+    # the built-in radii with a decimated term and a field: holes in a few blocks
+    ([2, 8, 32, 128], 5.0, (700, 1100), (160, 160, 380, 780), True, "disc", 0),
+    # the smallest blocks: some marked, their neighbours not
+    ([2, 8, 32], 10.0, (300, 700), (0, 0, 300, 700), False, "pixel", 8),
+    ([2, 8, 32], 10.0, (230, 431), (3, 0, 227, 430), False, "edge", 24),
+    # one and two radii, odd ones, remainders of strips and blocks
+    ([3], 10.0, (300, 517), (0, 0, 300, 517), False, "pixel", 0),
+    ([5, 21], 10.0, (411, 389), (0, 13, 400, 376), True, "scatter", 16),
+    ([2, 8, 30], 10.0, (257, 1000), (1, 3, 255, 990), True, "disc", 0),
+    # no valid sample at all; no NaN although the caller expects some; windows
+    # smaller than the widest radius
+    ([2, 8, 32], 10.0, (90, 300), (0, 0, 90, 300), False, "all", 0),
+    ([2, 8, 32], 10.0, (90, 300), (0, 0, 90, 300), False, "none", 0),
+    ([2, 8, 32], 10.0, (9, 7), (0, 0, 9, 7), False, "pixel", 8),
+    ([1], 10.0, (1, 1), (0, 0, 1, 1), False, "all", 0),
+])
+def test_wave_kernel_on_nan_windows(cuda, radii, px, shape, reg, field, holes, variant):
+    """A window with NaN: the wavefront kernel's plain blocks and the marked
+    ones' NaN-aware means give the workgroup kernel's bits."""
+    from fujishadergpu_amd import ops
+    from fujishadergpu_amd.algorithms import OutSpec, TopoUSMFastAlgorithm
+    from fujishadergpu_amd.encoding import quantize_params
+    H, W = shape
+    dem = _dem(max(H, 32), max(W, 32), 17 + H, relief=3776.0, hurst=0.75)[:H, :W].clone()
+    yy, xx = np.mgrid[0:H, 0:W]
+    if holes == "disc":
+        dem[torch.from_numpy((yy - H // 2) ** 2 + (xx - W // 3) ** 2 < (H // 6) ** 2)] = float("nan")
+    elif holes == "pixel":
+        dem[H // 2, W // 2] = float("nan")
+    elif holes == "edge":
+        dem[:, :40] = float("nan")
+        dem[-1, :] = float("nan")
+    elif holes == "scatter":
+        dem[torch.from_numpy(np.random.default_rng(3).random((H, W)) < 0.3)] = float("nan")
+    elif holes == "all":
+        dem[:] = float("nan")
+    g = dem.to(cuda)
+    p = dict(radii=radii, weights=[1.0 / len(radii)] * len(radii), pixel_size=px,
+             global_stats=(19.5,), _window_nan_free=False)
+    if field:
+        fld = ops.topousm_coarse_field(_dem(64, 96, 7, relief=3776.0, hurst=0.75).to(cuda),
+                                       [9], [0.03])
+        p.update(_topousm_fast_coarse_field=fld, _topousm_fast_small_radii=radii,
+                 _topousm_fast_small_weights=p["weights"], _topousm_fast_w_large=0.03,
+                 _topousm_fast_full_shape=(H * 3, W * 2), _topousm_fast_field_offset=(H, W // 2))
+    r0, c0, rh, rw = reg
+    qp = quantize_params(-1.176, 1.176, "uint8")
+    outs = []
+    try:
+        for v in (1, variant):
+            ops.set_topousm_variant(v)
+            f32 = torch.full((rh, rw), -7.0, dtype=torch.float32, device=cuda)
+            u8 = torch.zeros((rh, rw), dtype=torch.uint8, device=cuda)
+            TopoUSMFastAlgorithm().run_region(g, ops.region(r0, c0, rh, rw),
+                                              OutSpec(f32=f32, q=u8, qp=qp), p)
+            torch.cuda.synchronize()
+            outs.append((f32, u8))
+    finally:
+        ops.set_topousm_variant(0)
+    (a32, a8), (b32, b8) = outs
+    nan = torch.isnan(dem[r0:r0 + rh, c0:c0 + rw]).to(cuda)
+    assert torch.equal(torch.isnan(a32), nan) and torch.equal(torch.isnan(b32), nan)
+    assert torch.equal(torch.nan_to_num(a32), torch.nan_to_num(b32))
+    assert torch.equal(a8, b8)
+
+
 @pytest.mark.parametrize("h,w,dist,n_dirs,typ", [
     (384, 384, 50, 16, "positive"), (2304, 64, 64, 8, "negative"), (1153, 128, 8, 33, "positive"),
     (390, 389, 68, 3, "negative"), (385, 383, 69, 5, "positive"), (600, 257, 3, 1, "positive")])
