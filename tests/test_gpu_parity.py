@@ -566,6 +566,18 @@ def test_nodata_to_nan_and_counts(cuda):
     assert counts.cpu().tolist() == [2, 1]
 
 
+@pytest.mark.parametrize("h,w,ld", [(1, 1, 1), (3, 5, 9), (5, 1026, 1027), (2051, 37, 37),
+                                    (13, 4099, 4100)])
+def test_nan_counts_at_ragged_windows(cuda, h, w, ld):
+    from fujishadergpu_amd import ops
+    full = torch.rand(h, ld)
+    full[full < 0.3] = float("nan")
+    g = full.to(cuda)[:, :w]
+    wins = [(0, 0, h, w), (h // 2, w // 3, h - h // 2, w - w // 3), (0, w - 1, h, 1), (h - 1, 0, 1, w)]
+    counts = ops.nodata_to_nan(g, None, wins).cpu().tolist()
+    assert counts == [int(torch.isnan(full[r:r + hh, c:c + ww]).sum()) for r, c, hh, ww in wins]
+
+
 def test_row_mapped_launches_cover_rasters_taller_than_the_grid_limit(cuda):
     # 140001 rows (more than the 65535 blocks gridDim.y allows): NoData
     # conversion with a sentinel, region copy, encode and the block mean
