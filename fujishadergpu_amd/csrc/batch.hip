@@ -202,7 +202,7 @@ __global__ void __launch_bounds__(256) k_batch_rows(const RowsTile4* rt, const i
 
 // NaN-aware stencil tiles of a batch, one launch per tile.
 __global__ void __launch_bounds__(256) k_stencil_nanaw(StencilTile S, Gauss9 G) {
-  __shared__ float lds[ST_LDS_FLOATS_ROWS];
+  __shared__ __align__(16) float lds[ST_LDS_FLOATS_ROWS];
   stencil_tile_block<true>(S, blockIdx.y, blockIdx.x, G, lds);
 }
 

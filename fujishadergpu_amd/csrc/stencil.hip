@@ -50,7 +50,7 @@ __device__ __forceinline__ bool rect_block(const StencilTile& S, const RectSet& 
 // per-row x steps (larger LDS for the coefficient tables).
 template <bool NANAW, bool ROWS>
 __global__ void __launch_bounds__(256) k_stencil_tiles(StencilTile S, RectSet R, Gauss9 G) {
-  __shared__ float lds[ROWS ? ST_LDS_FLOATS_ROWS : ST_LDS_FLOATS];
+  __shared__ __align__(16) float lds[ROWS ? ST_LDS_FLOATS_ROWS : ST_LDS_FLOATS];
   StencilTile T;
   int bx, by;
   if (!rect_block(S, R, T, bx, by)) return;  // the whole block

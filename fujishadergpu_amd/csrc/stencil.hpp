@@ -56,6 +56,38 @@ __device__ __forceinline__ void nan_fill_col(const WinDev& W, int r, int cc, con
   fw = (float)sw;
 }
 
+// The axis-0 pass from the column's nine values, rows r - 4 .. r + 4 (clamped).
+__device__ __forceinline__ void nan_fill_sum(const float v[9], const Gauss9& G, float& fv,
+                                             float& fw) {
+  const bool v0 = !isnan(v[4]);
+  double sv = (v0 ? (double)v[4] : 0.0) * G.g[0];
+  double sw = (v0 ? 1.0 : 0.0) * G.g[0];
+#pragma unroll
+  for (int d = 4; d >= 1; d--) {
+    const float a = v[4 - d], b = v[4 + d];
+    const double fa = isnan(a) ? 0.0 : (double)a, fb = isnan(b) ? 0.0 : (double)b;
+    const double wa = isnan(a) ? 0.0 : 1.0, wb = isnan(b) ? 0.0 : 1.0;
+    sv += (fa + fb) * G.g[d];
+    sw += (wa + wb) * G.g[d];
+  }
+  fv = (float)sv;
+  fw = (float)sw;
+}
+
+// The axis-1 pass at ce from the column sums around it.
+__device__ __forceinline__ float nan_fill_row(const float2* ce, const Gauss9& G) {
+  double sv = (double)ce->x * G.g[0];
+  double sw = (double)ce->y * G.g[0];
+#pragma unroll
+  for (int d = 4; d >= 1; d--) {
+    const float2 a = ce[-d], b = ce[d];
+    sv += ((double)a.x + (double)b.x) * G.g[d];
+    sw += ((double)a.y + (double)b.y) * G.g[d];
+  }
+  const float fsv = (float)sv, fsw = (float)sw;
+  return fsw > 0.0f ? fsv / fsw : 0.0f;
+}
+
 // NaN-aware local fill at (r, c): scipy gaussian_filter(mode='nearest') of
 // filled*valid and of valid, axis 0 then axis 1 with float32 intermediates,
 // symmetric accumulation order (centre, then distance 4..1), then
@@ -333,8 +365,10 @@ __device__ __forceinline__ void stencil_tile_block_v(const StencilTile& S, int b
                                                      const Gauss9& G, float* lds) {
   const int rl = S.r0 + by * ST_TH, cl = S.c0 + bx * ST_TW;  // window coords of the block
   const int H = S.W.h, Wd = S.W.w;
-  const int tr0 = max(rl - ST_HALO, 0), tr1 = min(rl + ST_TH + ST_HALO, H);
-  const int tc0 = max(cl - ST_HALO, 0), tc1 = min(cl + ST_TW + ST_HALO, Wd);
+  // the block's outputs (the region may end inside it) and what they read
+  const int rows = min(ST_TH, S.rh - by * ST_TH), cols = min(ST_TW, S.rw - bx * ST_TW);
+  const int tr0 = max(rl - ST_HALO, 0), tr1 = min(rl + rows + ST_HALO, H);
+  const int tc0 = max(cl - ST_HALO, 0), tc1 = min(cl + cols + ST_HALO, Wd);
   const int nr = tr1 - tr0, nc = tc1 - tc0;
   float* F = lds;
   float* Pt = lds + ST_ROWS * ST_LT;
@@ -362,12 +396,46 @@ __device__ __forceinline__ void stencil_tile_block_v(const StencilTile& S, int b
         if (rr < nr && cc < nc) F[rr * ST_LT + cc] = v[i][j];
       }
     if (NANAW) {
-      // NaN cells (rare) take the local fill; one call site, the lane's own cells
+      // NaN cells take the local fill, both passes shared by the block: the
+      // column sums of NAN_ROWS staged rows and four columns either side in the
+      // derivative tables' space, then the block's NaN cells from those.  A
+      // block without a NaN cell, or without a valid output, needs none.  (Each
+      // lane filling its own cells walked 81 loads in turn per cell: the border
+      // strips of 1000 x 1531 cells with 1 % NoData 35 us, now 14.)
+      bool hole = false, valid = false;
+#pragma unroll
+      for (int i = 0; i < NRW; i++)
+#pragma unroll
+        for (int j = 0; j < NCW; j++) {
+          const int rr = (t >> 6) + 4 * i, cc = (t & 63) + 64 * j;
+          if (rr < nr && cc < nc) {
+            hole |= isnan(v[i][j]);
+            valid |= !isnan(v[i][j]) & (tr0 + rr >= rl) & (tr0 + rr < rl + rows) &
+                     (tc0 + cc >= cl) & (tc0 + cc < cl + cols);
+          }
+        }
+      if (__syncthreads_or(hole) && __syncthreads_or(valid)) {
+        constexpr int FW = ST_TW + 2 * ST_HALO + 8;             // column sums of a row
+        constexpr int NAN_ROWS = (2 * ST_PH * ST_PW) / (2 * FW);  // rows that fit
+        float2* sums = (float2*)Pt;
+        for (int b0 = 0; b0 < nr; b0 += NAN_ROWS) {
+          const int n = min(NAN_ROWS, nr - b0);
 #pragma unroll 1
-      for (int e = 0; e < NRW * NCW; e++) {
-        const int rr = (t >> 6) + 4 * (e / NCW), cc = (t & 63) + 64 * (e % NCW);
-        if (rr < nr && cc < nc && isnan(F[rr * ST_LT + cc]))
-          F[rr * ST_LT + cc] = nan_fill(S.W, tr0 + rr, tc0 + cc, G);
+          for (int e = t; e < n * FW; e += 256) {
+            const int rr = e / FW, cc = e - rr * FW;
+            float fv, fw;
+            nan_fill_col<false>(S.W, tr0 + b0 + rr, clampi(tc0 + cc - 4, Wd), G, fv, fw);
+            sums[e] = make_float2(fv, fw);
+          }
+          __syncthreads();
+#pragma unroll 1
+          for (int e = t; e < n * nc; e += 256) {
+            const int rr = e / nc, cc = e - rr * nc;
+            float* d = F + (b0 + rr) * ST_LT + cc;
+            if (isnan(*d)) *d = nan_fill_row(sums + rr * FW + cc + 4, G);
+          }
+          __syncthreads();
+        }
       }
     }
   }
@@ -395,7 +463,8 @@ __device__ __forceinline__ void stencil_tile_block_v(const StencilTile& S, int b
     for (int e = t; e < ST_PH * ST_PW; e += 256) {
       const int pr = e / ST_PW, pc = e - pr * ST_PW;
       const int i = rl - ST_RING + pr, j = cl - ST_RING + pc;
-      if (i >= 0 && i < H && j >= 0 && j < Wd) {
+      if (pr < rows + 2 * ST_RING && pc < cols + 2 * ST_RING && i >= 0 && i < H && j >= 0 &&
+          j < Wd) {
         Pt[e] = deriv(axr(i, ax), j, Wd, [&](int k) { return f(i, k); });
         Qt[e] = deriv(ay, i, H, [&](int k) { return f(k, j); });
       }

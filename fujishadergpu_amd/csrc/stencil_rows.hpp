@@ -129,18 +129,7 @@ __device__ __forceinline__ float wave_fill(const WinDev& W, int x, int c, int cb
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   float f = 0.0f;
-  if (want) {
-    double sv = (double)cv * G.g[0];
-    double sw = (double)cw * G.g[0];
-#pragma unroll
-    for (int d = 4; d >= 1; d--) {
-      const float2 a = cols[4 + lane - d], b = cols[4 + lane + d];
-      sv += ((double)a.x + (double)b.x) * G.g[d];
-      sw += ((double)a.y + (double)b.y) * G.g[d];
-    }
-    const float fsv = (float)sv, fsw = (float)sw;
-    f = fsw > 0.0f ? fsv / fsw : 0.0f;
-  }
+  if (want) f = nan_fill_row(cols + 4 + lane, G);
   // the next call overwrites the sums
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -341,23 +330,46 @@ __device__ __forceinline__ void load_group(const float* rowp, int c4, float z[4]
 // either side.
 constexpr int SR4_FILL_COLS = 264;
 
-// wave_fill for four columns per lane: the lane's four column sums (nine
-// loads each) and lanes 0..7 the four columns either side of the wave go to
-// LDS, then each wanted cell reads its nine in nan_fill's order, so the value
-// is nan_fill's bits.  z holds the raw row, want which cells need the fill;
-// the group's values come back in f (other NaN cells as 0: no output reads
-// them).  Every lane of the wave must call it.
+// wave_fill for four columns per lane: the column sums that the wanted cells
+// read go to LDS, then each wanted cell reads its nine in nan_fill's order, so
+// the value is nan_fill's bits.  Only the lanes with a wanted cell and their
+// neighbours form their four column sums (a cell reads four columns either
+// side, one lane's worth), from nine loads issued together; lanes 0..7 add
+// the four columns either side of the wave when its first or last lane wants one.  z holds the raw row, want which cells need the fill; the group's
+// values come back in f (other NaN cells as 0: no output reads them).  Every
+// lane of the wave must call it.  Bound: the latency of its loads and of the
+// float64 sums in the few waves that hold a void's edge.  Every lane loading 36
+// single values took a 4096^2 hillshade or slope launch from 61 us (no void) to 125
+// at 1 % NoData; now 109.  All 36 values of a lane in flight, or further rows
+// ahead in the walk, gained nothing and cost a wave per SIMD.
 __device__ __forceinline__ void wave_fill4(const WinDev& W, int x, int c4, int cb,
                                            const float z[4], const bool want[4],
                                            const Gauss9& G, float2* cols, float f[4]) {
   const int lane = threadIdx.x & 63;
+  const unsigned long long m =
+      __builtin_amdgcn_ballot_w64(want[0] | want[1] | want[2] | want[3]);
+  const unsigned long long need = m | (m << 1) | (m >> 1);
+  if ((need >> lane) & 1) {
+    // two columns at a time: 18 registers in flight (36 cost a wave per SIMD)
 #pragma unroll 1
-  for (int k = 0; k < 4; k++) {
-    float cv, cw;
-    nan_fill_col<false>(W, x, clampi(c4 + k, W.w), G, cv, cw);
-    cols[4 + 4 * lane + k] = make_float2(cv, cw);
+    for (int h = 0; h < 4; h += 2) {
+      float2 q[9];
+#pragma unroll
+      for (int d = -4; d <= 4; d++)
+        __builtin_memcpy(&q[d + 4], W.p + (int64_t)clampi(x + d, W.h) * W.ld + c4 + h,
+                         sizeof(float2));
+      float v[9], cv, cw;
+#pragma unroll
+      for (int d = 0; d < 9; d++) v[d] = q[d].x;
+      nan_fill_sum(v, G, cv, cw);
+      cols[4 + 4 * lane + h] = make_float2(cv, cw);
+#pragma unroll
+      for (int d = 0; d < 9; d++) v[d] = q[d].y;
+      nan_fill_sum(v, G, cv, cw);
+      cols[5 + 4 * lane + h] = make_float2(cv, cw);
+    }
   }
-  if (lane < 8) {
+  if (((m & 1) && lane < 4) || ((m >> 63) && lane >= 4 && lane < 8)) {
     const int col = lane < 4 ? cb - 4 + lane : cb + 256 + (lane - 4);
     float ev, ew;
     nan_fill_col<false>(W, x, clampi(col, W.w), G, ev, ew);
@@ -369,20 +381,7 @@ __device__ __forceinline__ void wave_fill4(const WinDev& W, int x, int c4, int c
 #pragma unroll
   for (int k = 0; k < 4; k++) {
     float v = isnan(z[k]) ? 0.0f : z[k];
-    if (want[k]) {
-      const int e = 4 + 4 * lane + k;
-      const float2 ce = cols[e];
-      double sv = (double)ce.x * G.g[0];
-      double sw = (double)ce.y * G.g[0];
-#pragma unroll
-      for (int d = 4; d >= 1; d--) {
-        const float2 a = cols[e - d], b = cols[e + d];
-        sv += ((double)a.x + (double)b.x) * G.g[d];
-        sw += ((double)a.y + (double)b.y) * G.g[d];
-      }
-      const float fsv = (float)sv, fsw = (float)sw;
-      v = fsw > 0.0f ? fsv / fsw : 0.0f;
-    }
+    if (want[k]) v = nan_fill_row(cols + 4 + 4 * lane + k, G);
     f[k] = v;
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -448,8 +447,10 @@ __device__ __forceinline__ bool rows4_wave(const RowsTile4& S, int& c4, int& cb,
 // Hillshade and/or slope, four columns per lane.  Rows arrive one per
 // iteration from ra - 1 on; the first two iterations only fill (so the NaN
 // fill has one call site).
+// (The bound of five waves per SIMD keeps the fill from taking more registers
+// than the walk: left alone it took 109, and four waves.)
 template <bool NANAW>
-__global__ void __launch_bounds__(256) k_shade_inner4(RowsTile4 S4, Gauss9 G) {
+__global__ void __launch_bounds__(256, NANAW ? 5 : 1) k_shade_inner4(RowsTile4 S4, Gauss9 G) {
   constexpr int LEFT = SR4_LEFT_SHADE;
   int c4, cb, ra, rb;
   if (!rows4_wave<LEFT>(S4, c4, cb, ra, rb)) return;  // the whole wave
@@ -549,7 +550,7 @@ __global__ void __launch_bounds__(256) k_shade_inner4(RowsTile4 S4, Gauss9 G) {
 // ra - 2 on; the first four iterations only build the rows' values and first
 // derivatives.
 template <bool NANAW>
-__global__ void __launch_bounds__(256) k_curv_inner4(RowsTile4 S4, Gauss9 G) {
+__global__ void __launch_bounds__(256, NANAW ? 5 : 1) k_curv_inner4(RowsTile4 S4, Gauss9 G) {
   constexpr int LEFT = SR4_LEFT_CURV;
   int c4, cb, ra, rb;
   if (!rows4_wave<LEFT>(S4, c4, cb, ra, rb)) return;  // the whole wave

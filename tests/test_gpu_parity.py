@@ -190,6 +190,49 @@ def _stencils_wide_windows(cuda, nan_discs, off, ld):
     _cmp("curvature/region", o_cv, ref_cv[sub], 4e-4)
 
 
+@pytest.mark.parametrize("h,w,holes", [
+    (203, 517, "discs"), (64, 300, "scatter"), (17, 1040, "edges"), (70, 259, "lines"),
+    (150, 390, "islands"),
+])
+def test_nan_fills_of_row_and_tile_kernels_agree(cuda, h, w, holes):
+    """The fill shared by a wave (row kernels) and by a block (tiled kernel),
+    against the oracle and against each other bit for bit: holes across tile
+    and wave edges, at the window's edges, isolated cells, isolated valid cells."""
+    from fujishadergpu_amd import ops
+    from fujishadergpu_amd.algorithms import ALGORITHMS
+    dem = _dem(max(h, 32), w, 5 + h, relief=1200.0)[:h].clone()
+    rng = np.random.default_rng(h)
+    yy, xx = np.mgrid[0:h, 0:w]
+    m = np.zeros((h, w), bool)
+    if holes == "discs":
+        for cy, cx, r in ((0, 0, 30), (100, 257, 45), (203, 517, 25), (60, 64, 3)):
+            m |= (yy - cy) ** 2 + (xx - cx) ** 2 <= r * r
+    elif holes == "scatter":
+        m = rng.random((h, w)) < 0.2
+    elif holes == "edges":
+        m[:2] = m[-1:] = True
+        m[:, :3] = m[:, -5:] = True
+    elif holes == "lines":
+        m[:, 60:70] = m[33:36] = m[:, 255:257] = True
+    else:
+        m[:] = rng.random((h, w)) < 0.98
+    dem[torch.from_numpy(m)] = float("nan")
+    g, a, kw = dem.to(cuda), dem.numpy(), dict(pixel_size=10.0)
+    got = {}
+    for split in (0, 1 << 40):
+        prev = ops.set_stencil_split_min(split)
+        try:
+            got[split] = [ALGORITHMS[k].process(g, **kw) for k in ("hillshade", "slope", "curvature")]
+        finally:
+            ops.set_stencil_split_min(prev)
+    for x, y in zip(got[0], got[1 << 40]):
+        assert torch.equal(torch.isnan(x), torch.isnan(y))
+        assert torch.equal(torch.nan_to_num(x), torch.nan_to_num(y))
+    _cmp("hillshade", got[0][0], ref.hillshade(a, **kw), 1e-6)
+    _cmp("slope", got[0][1], ref.slope(a, **kw), 2e-5, 1e-6)
+    _cmp("curvature", got[0][2], ref.curvature(a, curvature_type="mean", **kw), 4e-4)
+
+
 @pytest.mark.parametrize("radii,weights,px", [
     ([2, 8, 32], [0.5, 0.3, 0.2], 5.0),
     ([2, 8, 32, 128], [8 / 15, 4 / 15, 2 / 15, 1 / 15], 5.0),
