@@ -75,52 +75,80 @@ struct ConvArgs {
   int B, H, W, cin, kpad, cout;
 };
 
-template <int EPI>
-__global__ void __launch_bounds__(256) k_conv3x3(ConvArgs A) {
-  __shared__ __attribute__((aligned(16))) u16 wl[CNN_C * CNN_MAX_KPAD];
+// One 3x3 layer: C = W (32 out channels x K) * X (K x 32 pixels) a wave and
+// tile, with a tile 32 consecutive pixels of the flattened [B][H][W], so that no
+// tile is cut at a row's end and a tap is one offset for the whole wave; a
+// lane's edge tests are bits of its own.  Bound: memory (13 MB in, 13 out, 26
+// pre-activations at 32 x 80 x 80 cells: 11 us).  The channel count is a template
+// argument so that all of a tile's loads are in flight before its first
+// product (a loop over k-steps waited for each load in turn), and the weights'
+// LDS rows are 8 longer than K, whose 16-byte reads then spread over the banks
+// (32 -> 32 channels at those sizes: 28 us before, 22 now).  A wave takes equal shares of one resident round's tiles.
+constexpr int CONV_WAVES = 4096;   // four blocks of four waves a CU (128 registers)
+
+template <int EPI, int CIN>
+__global__ void __launch_bounds__(256, 4) k_conv3x3(ConvArgs A) {
+  constexpr int KS = (9 * CIN + 15) / 16;       // k-steps that reach a tap
+  __shared__ __attribute__((aligned(16))) u16 wl[CNN_C * (CNN_MAX_KPAD + 8)];
+  __shared__ __attribute__((aligned(16))) float bl[CNN_C];
   const int t = threadIdx.x;
-  const int nw = CNN_C * A.kpad;
-  for (int e = t * 8; e < nw; e += 256 * 8)
-    *(uint4*)(wl + e) = *(const uint4*)(A.wpack + e);
+  if (t < CNN_C) bl[t] = EPI != EPI_GELU_GRAD && t < A.cout ? A.bias[t] : 0.0f;
+  const int kp = A.kpad + 8;
+  for (int e = t * 8; e < CNN_C * A.kpad; e += 256 * 8) {
+    const int r = e / A.kpad;
+    *(uint4*)(wl + r * kp + (e - r * A.kpad)) = *(const uint4*)(A.wpack + e);
+  }
   __syncthreads();
-  const int lane = t & 63, wave = t >> 6;
+  const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int n = lane & 31, half = lane >> 5;
-  const int tiles_x = (A.W + 31) >> 5;
-  const int n_tiles = A.B * A.H * tiles_x;
-  const int ksteps = A.kpad >> 4;
-  // C = W (32 out channels x K) * X (K x 32 pixels): lane holds pixel n and
-  // channels 8i + half*4 + j at acc[4i + j]
-  float bias[16];
-#pragma unroll
-  for (int e = 0; e < 16; e++)
-    bias[e] = (EPI != EPI_GELU_GRAD && (8 * (e >> 2) + half * 4 + (e & 3)) < A.cout)
-                  ? A.bias[8 * (e >> 2) + half * 4 + (e & 3)]
-                  : 0.0f;
-  for (int tile = blockIdx.x * 4 + wave; tile < n_tiles; tile += gridDim.x * 4) {
-    const int tx = tile % tiles_x;
-    const int row = tile / tiles_x;  // b * H + y
-    const int b = row / A.H, y = row - b * A.H;
-    const int x0 = tx * 32;
-    const int px = x0 + n;           // this lane's pixel (B column)
-    f32x16 acc;   // starts at the bias: z = bias + sum_k w x
-#pragma unroll
-    for (int e = 0; e < 16; e++) acc[e] = bias[e];
-    for (int ks = 0; ks < ksteps; ks++) {
-      const int k = ks * 16 + half * 8;
-      const int tap = k / A.cin, ci = k - tap * A.cin;
-      bf16x8 a;
-      const int yy = y + tap / 3 - 1, xx = px + tap % 3 - 1;
-      if (tap < 9 && yy >= 0 && yy < A.H && xx >= 0 && xx < A.W) {
-        const uint4 v = *(const uint4*)(A.x + ((((int64_t)b * A.H + yy) * A.W + xx) * A.cin + ci));
-        a = __builtin_bit_cast(bf16x8, v);
-      } else {
-        a = __builtin_bit_cast(bf16x8, make_uint4(0, 0, 0, 0));
-      }
-      const bf16x8 w = __builtin_bit_cast(bf16x8, *(const uint4*)(wl + n * A.kpad + k));
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, a, acc, 0, 0, 0);
+  const int64_t n_px = (int64_t)A.B * A.H * A.W;
+  const int64_t n_tiles = (n_px + 31) >> 5;
+  const u16* wr = wl + n * kp + half * 8;
+  for (int64_t tile = (int64_t)blockIdx.x * 4 + wave; tile < n_tiles; tile += gridDim.x * 4) {
+    const int64_t p = tile * 32 + n;   // this lane's pixel (B column)
+    const bool in = p < n_px;
+    int x, y;
+    if (n_px <= 0x7fffffff) {
+      const unsigned row = (unsigned)p / (unsigned)A.W;
+      x = (int)((unsigned)p - row * (unsigned)A.W);
+      y = (int)(row % (unsigned)A.H);
+    } else {
+      const int64_t row = p / A.W;
+      x = (int)(p - row * A.W);
+      y = (int)(row % A.H);
     }
-    if (px >= A.W) continue;
-    const int64_t p = ((int64_t)b * A.H + y) * A.W + px;
+    // bit tap: the tap's pixel lies inside the patch
+    const int ym = (y > 0 ? 1 : 0) | 2 | (y < A.H - 1 ? 4 : 0);
+    const int xm = (x > 0 ? 1 : 0) | 2 | (x < A.W - 1 ? 4 : 0);
+    const int taps = in ? ((ym & 1) ? xm : 0) | (xm << 3) | ((ym & 4) ? xm << 6 : 0) : 0;
+    const u16* xp = A.x + tile * 32 * CIN;   // the whole wave's
+    const unsigned lo = n * CIN + (CIN == 8 ? 0 : half * 8);
+    uint4 v[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+      // CIN = 8: a k-step is two taps, one a half; CIN = 32: half a tap
+      const int tap = CIN == 8 ? 2 * ks + half : ks >> 1;
+      const int ci = CIN == 8 ? 0 : (ks & 1) * 16;
+      v[ks] = make_uint4(0, 0, 0, 0);
+      if ((taps >> tap) & 1)
+        v[ks] = *(const uint4*)(xp + ((int64_t)(tap / 3 - 1) * A.W + (tap % 3 - 1)) * CIN + ci + lo);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // lane holds pixel n and channels 8i + half*4 + j at acc[4i + j], which
+    // start at the bias: z = bias + sum_k w x
+    f32x16 acc;
+#pragma unroll
+    for (int e = 0; e < 16; e++) acc[e] = bl[8 * (e >> 2) + half * 4 + (e & 3)];
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++)
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+          __builtin_bit_cast(bf16x8, *(const uint4*)(wr + ks * 16)),
+          __builtin_bit_cast(bf16x8, v[ks]), acc, 0, 0, 0);
+    for (int k = KS * 16; k < A.kpad; k += 16)   // longer padding: zeros
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+          __builtin_bit_cast(bf16x8, *(const uint4*)(wr + k)),
+          __builtin_bit_cast(bf16x8, make_uint4(0, 0, 0, 0)), acc, 0, 0, 0);
+    if (!in) continue;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       const int c0 = 8 * i + half * 4;  // channels c0 .. c0 + 3
@@ -1028,23 +1056,26 @@ extern "C" int fsg_cnn_conv3x3(const fsg_cnn_conv* c, void* stream) {
     return fail(FSG_E_INVALID, "fsg_cnn_conv3x3: linear epilogue needs bias and yf");
   if (c->epilogue == FSG_CNN_GELU_GRAD && (!c->pre_in || !c->y))
     return fail(FSG_E_INVALID, "fsg_cnn_conv3x3: GELU-gradient epilogue needs pre_in and y");
-  const int64_t tiles = (int64_t)c->batch * c->h * ((c->w + 31) / 32);
-  const int grid = (int)std::min<int64_t>((tiles + 3) / 4, 256 * 16);
+  const int64_t tiles = ((int64_t)c->batch * c->h * c->w + 31) / 32;
+  const int64_t per = (tiles + CONV_WAVES - 1) / CONV_WAVES;
+  const dim3 grid((unsigned)((tiles + 4 * per - 1) / (4 * per))), blk(256);
   hipStream_t s = as_stream(stream);
   TimedScope ts("k_conv3x3", s);
+#define FSG_CONV_CASE(EPIV, NAME)                                                     \
+  case NAME:                                                                          \
+    if (c->cin == 8)                                                                  \
+      hipLaunchKernelGGL((k_conv3x3<EPIV, 8>), grid, blk, 0, s, A);                   \
+    else                                                                              \
+      hipLaunchKernelGGL((k_conv3x3<EPIV, 32>), grid, blk, 0, s, A);                  \
+    break;
   switch (c->epilogue) {
-    case FSG_CNN_GELU:
-      hipLaunchKernelGGL(k_conv3x3<EPI_GELU>, dim3(grid), dim3(256), 0, s, A);
-      break;
-    case FSG_CNN_LINEAR:
-      hipLaunchKernelGGL(k_conv3x3<EPI_LINEAR>, dim3(grid), dim3(256), 0, s, A);
-      break;
-    case FSG_CNN_GELU_GRAD:
-      hipLaunchKernelGGL(k_conv3x3<EPI_GELU_GRAD>, dim3(grid), dim3(256), 0, s, A);
-      break;
+    FSG_CONV_CASE(EPI_GELU, FSG_CNN_GELU)
+    FSG_CONV_CASE(EPI_LINEAR, FSG_CNN_LINEAR)
+    FSG_CONV_CASE(EPI_GELU_GRAD, FSG_CNN_GELU_GRAD)
     default:
       return fail(FSG_E_INVALID, "fsg_cnn_conv3x3: bad epilogue");
   }
+#undef FSG_CONV_CASE
   FSG_CHECK_LAUNCH("k_conv3x3");
   return FSG_OK;
 }

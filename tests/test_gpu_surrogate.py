@@ -147,6 +147,51 @@ def test_wgrad_at_strip_and_row_group_edges(cuda, cin, bsz, h, w):
                                            s))
 
 
+@pytest.mark.parametrize("cin,kpad", [(8, 80), (8, 96), (32, 288)])
+@pytest.mark.parametrize("bsz,h,w", [(1, 1, 1), (1, 1, 33), (2, 5, 3), (1, 7, 31), (3, 4, 32),
+                                     (1, 2, 97), (40, 61, 57)])
+def test_conv_layer_at_tile_and_patch_edges(cuda, cin, kpad, bsz, h, w):
+    """One layer against float64 where 32-pixel tiles span rows and patches, in one pixel
+    and in more tiles than a round of waves.  Float32 sums of n products (and the bias)
+    are off by at most n 2^-24 times the sum of their magnitudes; the three epilogues see
+    the same sums."""
+    import ctypes as C
+    from fujishadergpu_amd import _native as N
+    g = torch.Generator(device=cuda).manual_seed(11)
+    x = torch.randn((bsz, h, w, cin), generator=g, device=cuda).to(torch.bfloat16)
+    wt = torch.zeros((32, kpad), device=cuda)
+    wt[:, :9 * cin] = torch.randn((32, 9 * cin), generator=g, device=cuda)
+    wt = wt.to(torch.bfloat16)
+    bias = torch.randn(32, generator=g, device=cuda)
+    zero = torch.zeros(32, device=cuda)
+    xp = torch.nn.functional.pad(x.double(), (0, 0, 1, 1, 1, 1))
+    cols = torch.cat([xp[:, t // 3:t // 3 + h, t % 3:t % 3 + w] for t in range(9)], dim=3)
+    cols, wd = cols.reshape(-1, 9 * cin), wt[:, :9 * cin].double()
+    ref, mag = cols @ wd.T + bias.double(), cols.abs() @ wd.abs().T + bias.abs().double()
+    s = torch.cuda.current_stream().cuda_stream
+
+    def run(epi, b, cout=32, **bufs):
+        c = N.fsg_cnn_conv()
+        c.x, c.wpack, c.bias = x.data_ptr(), wt.data_ptr(), b.data_ptr()
+        c.batch, c.h, c.w, c.cin, c.kpad, c.cout, c.epilogue = bsz, h, w, cin, kpad, cout, epi
+        for k, v in bufs.items():
+            setattr(c, k, v.data_ptr())
+        N.check(N.lib().fsg_cnn_conv3x3(C.byref(c), s))
+
+    f = [torch.full((bsz * h * w, 32), -9.0, device=cuda) for _ in range(4)]
+    y = [torch.zeros((bsz * h * w, 32), dtype=torch.bfloat16, device=cuda) for _ in range(2)]
+    run(N.CNN_LINEAR, bias, yf=f[0])
+    run(N.CNN_GELU, bias, y=y[0], pre_out=f[1])
+    run(N.CNN_LINEAR, zero, yf=f[2])
+    run(N.CNN_GELU_GRAD, zero, y=y[1], pre_in=torch.full_like(f[3], 50.0))   # gelu' = 1
+    assert bool(((f[0].double() - ref).abs() <= (9 * cin + 1) * 2.0 ** -24 * mag).all())
+    assert torch.equal(f[0], f[1])
+    assert torch.equal(y[1], f[2].to(torch.bfloat16))
+    one = torch.full((bsz * h * w, 1), -9.0, device=cuda)
+    run(N.CNN_LINEAR, bias, cout=1, yf=one)
+    assert torch.equal(one[:, 0], f[0][:, 0])
+
+
 @pytest.mark.parametrize("f", [8, 4, 16])
 def test_compose_and_detail_label_match_the_oracle(cuda, f):
     from fujishadergpu_amd import _native as N
