@@ -83,7 +83,8 @@ struct ConvArgs {
 // argument so that all of a tile's loads are in flight before its first
 // product (a loop over k-steps waited for each load in turn), and the weights'
 // LDS rows are 8 longer than K, whose 16-byte reads then spread over the banks
-// (32 -> 32 channels at those sizes: 28 us before, 22 now).  A wave takes equal shares of one resident round's tiles.
+// (32 -> 32 channels at those sizes: 28 us before, 22 now).  A wave takes equal
+// shares of one resident round's tiles.
 constexpr int CONV_WAVES = 4096;   // four blocks of four waves a CU (128 registers)
 
 template <int EPI, int CIN>

@@ -113,8 +113,8 @@ __global__ void __launch_bounds__(256) k_shade_rows(StencilTile S0, RectSet R, G
   }
 }
 
-// Windows with NaN: one lane per pixel (the fill inlined at each neighbour
-// read takes the registers that a row walk would need).
+// The border strips of windows with NaN: one lane per pixel (the fill inlined at
+// each neighbour read takes the registers that a row walk would need).
 template <bool NANAW>
 __global__ void __launch_bounds__(256) k_shade_px(StencilTile S0, RectSet R, Gauss9 G) {
   StencilTile S;
@@ -206,13 +206,13 @@ static RowsTile rows_tile(const StencilTile& S, const fsg_region* reg, const Rec
 // The general kernels (every position, numpy's edge formulas included) over
 // up to RS_MAX rectangles of the region, one launch: hillshade/slope (one
 // lane per pixel with NaN, a row walk without) or curvature (tiled block).
-static void launch_general(const StencilTile& S, const Rect* q, int n, bool curv,
+static void launch_general(const StencilTile& S, const Rect* q, int n, bool tiled,
                            hipStream_t s) {
-  const int bh = curv ? ST_TH : (S.nanaw ? 4 : 4 * SHADE_R);
+  const int bh = tiled ? ST_TH : (S.nanaw ? 4 : 4 * SHADE_R);
   const RectSet R = rect_set(q, n, bh);
   if (R.n == 0) return;
   const dim3 grd((unsigned)R.pre[R.n]);
-  if (curv) {
+  if (tiled) {
     if (S.nanaw)
       hipLaunchKernelGGL((k_stencil_tiles<true, false>), grd, dim3(256), 0, s, S, R, make_gauss9());
     else
@@ -230,9 +230,8 @@ static void launch_general(const StencilTile& S, const Rect* q, int n, bool curv
 // hide its loads (2048^2 windows ran faster as one general launch).
 constexpr int64_t SPLIT_MIN_DEFAULT = int64_t(1) << 23;
 static std::atomic<int64_t> g_split_min{SPLIT_MIN_DEFAULT};
-// NaN-aware windows: the general kernel's fill is far slower than the row
-// kernels' wave fill, so their interiors take the row kernels from 2^20
-// pixels (or the process-wide setting, when smaller).
+// NaN-aware windows take the row kernels from 2^20 interior pixels (or the
+// process-wide setting, when smaller).
 constexpr int64_t SPLIT_MIN_NANAW = int64_t(1) << 20;
 
 // Constant-step hillshade/slope or curvature: the row-walking kernel over
@@ -309,7 +308,7 @@ static void launch_split(const StencilTile& S, const fsg_window* win, const fsg_
   } else {
     gen[ng++] = Rect{reg->r0, reg->c0, reg->h, reg->w};
   }
-  launch_general(S, gen, ng, curv, s);
+  launch_general(S, gen, ng, curv || (S.nanaw && !ok), s);
 }
 
 static StencilTile stencil_tile(const fsg_window* win, const fsg_region* reg) {

@@ -326,67 +326,76 @@ __device__ __forceinline__ void load_group(const float* rowp, int c4, float z[4]
   z[3] = t.w;
 }
 
-// Column sums the four-column wave fill keeps per wave: 256 columns and 4
-// either side.
-constexpr int SR4_FILL_COLS = 264;
+// What the four-column wave fill keeps per wave in LDS: the column sums of its
+// 256 columns and 4 either side (groups of four: group e covers columns 4e - 4 ..
+// 4e - 1 of the wave), the groups to sum, the cells to fill and their values.
+struct Fill4 {
+  float2 cols[264];
+  float out[256];
+  unsigned char cell[256];
+  unsigned char grp[72];
+};
 
-// wave_fill for four columns per lane: the column sums that the wanted cells
-// read go to LDS, then each wanted cell reads its nine in nan_fill's order, so
-// the value is nan_fill's bits.  Only the lanes with a wanted cell and their
-// neighbours form their four column sums (a cell reads four columns either
-// side, one lane's worth), from nine loads issued together; lanes 0..7 add
-// the four columns either side of the wave when its first or last lane wants one.  z holds the raw row, want which cells need the fill; the group's
-// values come back in f (other NaN cells as 0: no output reads them).  Every
-// lane of the wave must call it.  Bound: the latency of its loads and of the
-// float64 sums in the few waves that hold a void's edge.  Every lane loading 36
-// single values took a 4096^2 hillshade or slope launch from 61 us (no void) to 125
-// at 1 % NoData; now 109.  All 36 values of a lane in flight, or further rows
-// ahead in the walk, gained nothing and cost a wave per SIMD.
-__device__ __forceinline__ void wave_fill4(const WinDev& W, int x, int c4, int cb,
-                                           const float z[4], const bool want[4],
-                                           const Gauss9& G, float2* cols, float f[4]) {
-  const int lane = threadIdx.x & 63;
-  const unsigned long long m =
-      __builtin_amdgcn_ballot_w64(want[0] | want[1] | want[2] | want[3]);
-  const unsigned long long need = m | (m << 1) | (m >> 1);
-  if ((need >> lane) & 1) {
-    // two columns at a time: 18 registers in flight (36 cost a wave per SIMD)
-#pragma unroll 1
-    for (int h = 0; h < 4; h += 2) {
-      float2 q[9];
-#pragma unroll
-      for (int d = -4; d <= 4; d++)
-        __builtin_memcpy(&q[d + 4], W.p + (int64_t)clampi(x + d, W.h) * W.ld + c4 + h,
-                         sizeof(float2));
-      float v[9], cv, cw;
-#pragma unroll
-      for (int d = 0; d < 9; d++) v[d] = q[d].x;
-      nan_fill_sum(v, G, cv, cw);
-      cols[4 + 4 * lane + h] = make_float2(cv, cw);
-#pragma unroll
-      for (int d = 0; d < 9; d++) v[d] = q[d].y;
-      nan_fill_sum(v, G, cv, cw);
-      cols[5 + 4 * lane + h] = make_float2(cv, cw);
-    }
-  }
-  if (((m & 1) && lane < 4) || ((m >> 63) && lane >= 4 && lane < 8)) {
-    const int col = lane < 4 ? cb - 4 + lane : cb + 256 + (lane - 4);
-    float ev, ew;
-    nan_fill_col<false>(W, x, clampi(col, W.w), G, ev, ew);
-    cols[lane < 4 ? lane : 256 + lane] = make_float2(ev, ew);
-  }
+// Lanes below this one whose bit is set.
+__device__ __forceinline__ int lanes_below(unsigned long long b) {
+  return __builtin_amdgcn_mbcnt_hi((unsigned)(b >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)b, 0));
+}
+
+__device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// wave_fill for four columns per lane.  z holds the raw row, want which cells need
+// the fill; the group's values come back in f (other NaN cells as 0: no output
+// reads them).  Every lane of the wave must call it.
+// Few cells of a row want the fill (a void's edge), so the work is dealt out
+// anew: the column sums that they read, a group of four columns (the reach of
+// the axis-1 pass is one group either side) to four lanes, then a cell to a lane, each
+// in nan_fill's order, so the value is nan_fill's bits.  Bound: the float64
+// sums of the waves at a void's edge, which share a few SIMDs.  With every lane
+// summing its own four columns a 4096^2 curvature launch took 133 us at 1 % NoData
+// (80 without a void), hillshade or slope 108 (58); now 113 and 99.
+__device__ __forceinline__ void wave_fill4(const WinDev& W, int x, int cb, const float z[4],
+                                           const bool want[4], const Gauss9& G, Fill4& L,
+                                           float f[4]) {
+  const int lane = threadIdx.x & 63;
+  unsigned long long m = 0;
+  int n_cells = 0;
 #pragma unroll
   for (int k = 0; k < 4; k++) {
-    float v = isnan(z[k]) ? 0.0f : z[k];
-    if (want[k]) v = nan_fill_row(cols + 4 + 4 * lane + k, G);
-    f[k] = v;
+    const unsigned long long b = __builtin_amdgcn_ballot_w64(want[k]);
+    if (want[k]) L.cell[n_cells + lanes_below(b)] = (unsigned char)(4 * lane + k);
+    n_cells += __popcll(b);
+    m |= b;
   }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  // groups 1 .. 64 are the lanes' own; 0 and 65 lie either side of the wave
+  const unsigned long long need = m | (m << 1) | (m >> 1);
+  const int left = (int)(m & 1), right = (int)(m >> 63);
+  if ((need >> lane) & 1) L.grp[left + lanes_below(need)] = (unsigned char)(lane + 1);
+  const int n_own = left + __popcll(need), n_grp = n_own + right;
+  if (lane == 0 && left) L.grp[0] = 0;
+  if (lane == 0 && right) L.grp[n_own] = 65;
+  wave_lds_sync();
+#pragma unroll 1
+  for (int g = lane >> 2; g < n_grp; g += 16) {
+    const int e = 4 * (int)L.grp[g] + (lane & 3);
+    float cv, cw;
+    nan_fill_col<false>(W, x, clampi(cb - 4 + e, W.w), G, cv, cw);
+    L.cols[e] = make_float2(cv, cw);
+  }
+  wave_lds_sync();
+#pragma unroll 1
+  for (int i = lane; i < n_cells; i += 64) {
+    const int c = L.cell[i];
+    L.out[c] = nan_fill_row(L.cols + 4 + c, G);
+  }
+  wave_lds_sync();
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+    f[k] = want[k] ? L.out[4 * lane + k] : (isnan(z[k]) ? 0.0f : z[k]);
+  wave_lds_sync();   // the next call overwrites them
 }
 
 // Writes v[0..3] at output row orr, columns occ .. occ+3 where ok[k] is set.
@@ -447,10 +456,10 @@ __device__ __forceinline__ bool rows4_wave(const RowsTile4& S, int& c4, int& cb,
 // Hillshade and/or slope, four columns per lane.  Rows arrive one per
 // iteration from ra - 1 on; the first two iterations only fill (so the NaN
 // fill has one call site).
-// (The bound of five waves per SIMD keeps the fill from taking more registers
-// than the walk: left alone it took 109, and four waves.)
+// (The bound of six waves per SIMD keeps the fill from taking more registers
+// than the walk; five ran 3 % slower at 1 % NoData.)
 template <bool NANAW>
-__global__ void __launch_bounds__(256, NANAW ? 5 : 1) k_shade_inner4(RowsTile4 S4, Gauss9 G) {
+__global__ void __launch_bounds__(256, NANAW ? 6 : 1) k_shade_inner4(RowsTile4 S4, Gauss9 G) {
   constexpr int LEFT = SR4_LEFT_SHADE;
   int c4, cb, ra, rb;
   if (!rows4_wave<LEFT>(S4, c4, cb, ra, rb)) return;  // the whole wave
@@ -479,27 +488,30 @@ __global__ void __launch_bounds__(256, NANAW ? 5 : 1) k_shade_inner4(RowsTile4 S
   rowp += (1 + AHEAD) * ld;  // row ra + AHEAD
   float fu[4] = {0.f, 0.f, 0.f, 0.f}, fm[4] = {0.f, 0.f, 0.f, 0.f};
   float zm[4] = {0.f, 0.f, 0.f, 0.f};
-  __shared__ float2 fill_cols[4][SR4_FILL_COLS];
+  __shared__ Fill4 fill[4];
   for (int r = ra - 2; r < rb; r++) {
     float fd[4] = {zd[0], zd[1], zd[2], zd[3]};
     if (NANAW) {
       // a NaN cell of row r + 1 is filled when an output reading it is valid:
-      // (r, c), (r + 2, c), (r + 1, c -+ 1); every lane takes part in the shifts
-      const float zl = lane_left(zd[3]), zr = lane_right(zd[0]);
-      bool want[4];
-      bool any_want = false;
+      // (r, c), (r + 2, c), (r + 1, c -+ 1); every lane takes part in the shifts.
+      // Most rows of most waves hold none
+      if (__ballot(isnan(zd[0]) | isnan(zd[1]) | isnan(zd[2]) | isnan(zd[3]))) {
+        const float zl = lane_left(zd[3]), zr = lane_right(zd[0]);
+        bool want[4];
+        bool any_want = false;
 #pragma unroll
-      for (int k = 0; k < 4; k++) {
-        const float left = k == 0 ? zl : zd[k - 1], right = k == 3 ? zr : zd[k + 1];
-        want[k] = isnan(zd[k]) & (!isnan(zm[k]) | !isnan(zq[0][k]) | !isnan(left) |
-                                  !isnan(right));
-        any_want |= want[k];
+        for (int k = 0; k < 4; k++) {
+          const float left = k == 0 ? zl : zd[k - 1], right = k == 3 ? zr : zd[k + 1];
+          want[k] = isnan(zd[k]) & (!isnan(zm[k]) | !isnan(zq[0][k]) | !isnan(left) |
+                                    !isnan(right));
+          any_want |= want[k];
+        }
+        if (__ballot(any_want))  // the whole wave
+          wave_fill4(S.W, r + 1, cb, zd, want, G, fill[threadIdx.x >> 6], fd);
+        else
+#pragma unroll
+          for (int k = 0; k < 4; k++) fd[k] = isnan(zd[k]) ? 0.0f : zd[k];
       }
-      if (__ballot(any_want))  // the whole wave
-        wave_fill4(S.W, r + 1, c4, cb, zd, want, G, fill_cols[threadIdx.x >> 6], fd);
-      else
-#pragma unroll
-        for (int k = 0; k < 4; k++) fd[k] = isnan(zd[k]) ? 0.0f : zd[k];
     }
     const float fl = lane_left(fm[3]), fr = lane_right(fm[0]);
     if (r >= ra && any) {
@@ -585,33 +597,36 @@ __global__ void __launch_bounds__(256, NANAW ? 5 : 1) k_curv_inner4(RowsTile4 S4
   float pm[4] = {0.f, 0.f, 0.f, 0.f}, p0[4] = {0.f, 0.f, 0.f, 0.f};
   float qm[4] = {0.f, 0.f, 0.f, 0.f}, q0[4] = {0.f, 0.f, 0.f, 0.f};
   float zc[4] = {0.f, 0.f, 0.f, 0.f}, zc1[4] = {0.f, 0.f, 0.f, 0.f};
-  __shared__ float2 fill_cols[4][SR4_FILL_COLS];
+  __shared__ Fill4 fill[4];
   for (int r = ra - 4; r < rb; r++) {
     float f4[4] = {zn[0], zn[1], zn[2], zn[3]}, pp[4], qp[4];
     if (NANAW) {
       // a NaN cell of row r + 2 is filled when a valid cell lies within two
-      // rows and two columns of it (the reach of the derivatives reading it)
-      int colv = 0;
+      // rows and two columns of it (the reach of the derivatives reading it);
+      // most rows of most waves hold none
+      if (__ballot(isnan(zn[0]) | isnan(zn[1]) | isnan(zn[2]) | isnan(zn[3]))) {
+        int colv = 0;
 #pragma unroll
-      for (int k = 0; k < 4; k++)
-        colv |= (!isnan(zc[k]) | !isnan(zc1[k]) | !isnan(zn[k]) | !isnan(zq[0][k]) |
-                 !isnan(zq[1][k])) << k;
-      // the neighbour lanes' masks; outside the wave counts as valid
-      const int ml = __builtin_amdgcn_update_dpp(0xf, colv, 0x138, 0xf, 0xf, false);
-      const int mr = __builtin_amdgcn_update_dpp(0xf, colv, 0x130, 0xf, 0xf, false);
-      const int w12 = ml | (colv << 4) | (mr << 8);  // columns c4 - 4 .. c4 + 7
-      bool want[4];
-      bool any_want = false;
+        for (int k = 0; k < 4; k++)
+          colv |= (!isnan(zc[k]) | !isnan(zc1[k]) | !isnan(zn[k]) | !isnan(zq[0][k]) |
+                   !isnan(zq[1][k])) << k;
+        // the neighbour lanes' masks; outside the wave counts as valid
+        const int ml = __builtin_amdgcn_update_dpp(0xf, colv, 0x138, 0xf, 0xf, false);
+        const int mr = __builtin_amdgcn_update_dpp(0xf, colv, 0x130, 0xf, 0xf, false);
+        const int w12 = ml | (colv << 4) | (mr << 8);  // columns c4 - 4 .. c4 + 7
+        bool want[4];
+        bool any_want = false;
 #pragma unroll
-      for (int k = 0; k < 4; k++) {
-        want[k] = isnan(zn[k]) & (((w12 >> (k + 2)) & 0x1f) != 0);
-        any_want |= want[k];
+        for (int k = 0; k < 4; k++) {
+          want[k] = isnan(zn[k]) & (((w12 >> (k + 2)) & 0x1f) != 0);
+          any_want |= want[k];
+        }
+        if (__ballot(any_want))  // the whole wave
+          wave_fill4(S.W, r + 2, cb, zn, want, G, fill[threadIdx.x >> 6], f4);
+        else
+#pragma unroll
+          for (int k = 0; k < 4; k++) f4[k] = isnan(zn[k]) ? 0.0f : zn[k];
       }
-      if (__ballot(any_want))  // the whole wave
-        wave_fill4(S.W, r + 2, c4, cb, zn, want, G, fill_cols[threadIdx.x >> 6], f4);
-      else
-#pragma unroll
-        for (int k = 0; k < 4; k++) f4[k] = isnan(zn[k]) ? 0.0f : zn[k];
     }
     const float l1 = lane_left(fi1[3]), r1 = lane_right(fi1[0]);
     const float lp = lane_left(p0[3]), rp = lane_right(p0[0]);
