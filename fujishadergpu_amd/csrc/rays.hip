@@ -3,8 +3,8 @@
 // Openness (compute_openness_vectorized, _impl_openness.py:31-132): per
 // direction the horizon extreme of atan((z_s - z) / d) over the valid
 // in-window samples.  atan is monotone, so the kernel takes the extreme of the
-// slope ratio, and the directions' angles are summed as the argument of a
-// product of complex numbers (AngleSum): one atan per pixel.
+// slope ratio and evaluates one atanf per direction instead of one per sample
+// (AngleSum).
 // The ratio uses f32(1/phys) multiplication (within 1.5 ulp of the reference's
 // division by f32(phys)).
 //
@@ -77,7 +77,7 @@ k_openness(WinDevR W, int r0, int c0, int rh, int rw, OpenTab T, OutDev out, Ray
     store_out(out, r, c, apply_post(pp, __builtin_nanf("")));
     return;
   }
-  double a;
+  float a;
   if constexpr (ND > 0)
     a = !interior ? openness_angle_u<ND, true>(W, i, j, z, T)
         : open_off32(W, T) ? openness_angle_u<ND, false, true>(W, i, j, z, T)
@@ -209,7 +209,7 @@ __device__ __forceinline__ const float* lds_sample(const char* at, short2 off) {
 // openness_angle_s, so the same bits.
 template <int ND, bool NEG>
 __device__ __forceinline__ void openness_pair(const char* at, const float z[2], const OpenTab& T,
-                                              double out[2]) {
+                                              float out[2]) {
   AngleSum S[2];
   for (int d = 0; d < T.n_dirs; d++) {
     float v[ND][2];
@@ -235,18 +235,12 @@ __device__ __forceinline__ void openness_pair(const char* at, const float z[2], 
       S[1].add<NEG>(ext[1]);
     } else {
 #pragma unroll
-      for (int m = 0; m < 2; m++) {
-        if (isnan(ext[m])) S[m].missing++;
-        else S[m].add<NEG>(ext[m]);
-      }
-    }
-    if ((d & 3) == 3) {
-      S[0].rescale();
-      S[1].rescale();
+      for (int m = 0; m < 2; m++)
+        if (!isnan(ext[m])) S[m].add<NEG>(ext[m]);
     }
   }
-  out[0] = S[0].mean(T);
-  out[1] = S[1].mean(T);
+  out[0] = S[0].mean();
+  out[1] = S[1].mean();
 }
 
 template <int ND>
@@ -267,7 +261,7 @@ k_openness_tile(WinDevR W, int r0, int c0, int rh, int rw, OpenTab T, RayTile R,
     const float z[2] = {at[0], at[64]};
     // a NaN pixel's ratios would all be NaN (and its columns past the window too)
     const float zv[2] = {isnan(z[0]) ? 0.0f : z[0], isnan(z[1]) ? 0.0f : z[1]};
-    double a[2];
+    float a[2];
     if (T.negative)
       openness_pair<ND, true>((const char*)at, zv, T, a);
     else
@@ -411,7 +405,7 @@ struct AoTab {
 // to [0, 1] (so within [0, pi/4]; 0 for a NaN sample), the argument of 1 + i
 // ratio, and arguments add under multiplication.  A group's product has its
 // argument within [0, pi]; the running product is kept in the upper half plane
-// like AngleSum's, with the half turns counted, so a run of any length takes one
+// with the half turns counted, so a run of any length takes one
 // atan: two FMAs and an eighth of a complex product more a sample in place of
 // an atanf, a division and a mask.
 struct AoRun {

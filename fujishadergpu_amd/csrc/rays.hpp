@@ -23,7 +23,6 @@ struct OpenTab {
   int negative;
   int raw;         // 1: mean angle in degrees instead of the display value
   int dmax_y, dmax_x;  // largest |offset| on each axis (interior test)
-  double inv_dirs; // 1 / n_dirs
   short2 off[OPEN_MAX];
   float inv[OPEN_MAX];
 };
@@ -71,48 +70,28 @@ __device__ __forceinline__ float gamma_pow(double z) {
 }
 
 // Sum over directions of the angle from the zenith (positive openness) or the
-// nadir, pi/2 - atan(e) of the direction's extreme ratio e (pi/2 + atan(e) when
-// negative), without an atan per direction: the angle is arg(e + i), and
-// arguments add under multiplication.  The running product x + i |y| is kept in
-// the upper half plane -- a factor turns it by less than pi, so where its
-// imaginary part comes out negative the product is negated and one half turn
-// counted -- and scaled by a power of two every fourth factor.  |e| is limited
-// to 2^28, where the angle is within 4e-9 of its limit.  Five operations a
-// direction and one atan a pixel, where an atan a direction took about 40 of
-// 100 operations; the float64 sum of half turns and remainder also rounds less
-// often than a float32 sum of angles did (8192 x 6144, 16 directions, relative to
-// float64 results: 7e-7 to 9e-7 then, 4e-7 to 5e-7 now).
+// nadir, in float32 as the reference adds them: pi/2 - atan(e) of the direction's
+// extreme ratio e (pi/2 + atan(e) when negative).  (arg of the product of e + i
+// over the directions is nearer the float64 results and took an 8192 x 6144 job
+// from 2795 to 2409 us, but moves more 8-bit display values of a flat raster than
+// their rounding allows.)
 struct AngleSum {
-  float x = 1.0f, y = 0.0f;   // y: its sign is not part of the value
-  unsigned signs = 0;         // negations since the last rescale, one bit each
-  int turns = 0, missing = 0; // half turns; directions without a valid sample
+  float sum = 0.0f;
+  int dirs = 0;
   template <bool NEG>
   __device__ __forceinline__ void add(float ext) {
-    const float e = __builtin_amdgcn_fmed3f(NEG ? -ext : ext, -0x1p28f, 0x1p28f);
-    const float nx = __builtin_fmaf(x, e, -fabsf(y)), ny = __builtin_fmaf(fabsf(y), e, x);
-    x = __uint_as_float(__float_as_uint(nx) ^ (__float_as_uint(ny) & 0x80000000u));
-    y = ny;
-    signs = __builtin_amdgcn_alignbit(signs, __float_as_uint(ny), 31);
-  }
-  __device__ __forceinline__ void rescale() {
-    const int e = -__builtin_amdgcn_frexp_expf(fmaxf(fabsf(x), fabsf(y)));
-    x = ldexpf(x, e);
-    y = ldexpf(y, e);
-    turns += __popc(signs);
-    signs = 0;
+    const float a = atanf(ext);
+    sum = sum + (NEG ? 1.57079637f + a : 1.57079637f - a);
+    dirs++;
   }
   // mean over the directions added (0 without any)
-  __device__ __forceinline__ double mean(const OpenTab& T) const {
-    const double sum = __builtin_fma((double)(turns + __popc(signs)), M_PI,
-                                     (double)arg_upper(x, fabsf(y)));
-    return sum * (missing == 0 ? T.inv_dirs : 1.0 / (double)max(T.n_dirs - missing, 1));
-  }
+  __device__ __forceinline__ float mean() const { return sum / fmaxf((float)dirs, 1.0f); }
 };
 
 // Mean openness angle (radians) at window (i, j): per direction the extreme
 // elevation ratio over its samples, averaged over the directions that saw a
 // valid sample (_impl_openness.py:78-126).
-__device__ __forceinline__ double openness_angle(const WinDevR& W, int i, int j, float z,
+__device__ __forceinline__ float openness_angle(const WinDevR& W, int i, int j, float z,
                                                 const OpenTab& T) {
   AngleSum S;
   for (int d = 0; d < T.n_dirs; d++) {
@@ -130,12 +109,11 @@ __device__ __forceinline__ double openness_angle(const WinDevR& W, int i, int j,
       ext = T.negative ? fminf(ext, q) : fmaxf(ext, q);
       any = true;
     }
-    if (!any) S.missing++;
-    else if (T.negative) S.add<true>(ext);
+    if (!any) continue;
+    if (T.negative) S.add<true>(ext);
     else S.add<false>(ext);
-    if ((d & 3) == 3) S.rescale();
   }
-  return S.mean(T);
+  return S.mean();
 }
 
 // The same angle with the distances of a direction unrolled (n_dist <= 10,
@@ -155,7 +133,7 @@ __device__ __forceinline__ double openness_angle(const WinDevR& W, int i, int j,
 constexpr int OPEN_UNROLL = 10;
 
 template <int ND, bool CHECK, bool OFF32, bool NEG>
-__device__ __forceinline__ double openness_angle_s(const WinDevR& W, int i, int j, float z,
+__device__ __forceinline__ float openness_angle_s(const WinDevR& W, int i, int j, float z,
                                                   const OpenTab& T) {
   // ND = 10: the table row of a direction is a fixed 10 entries (wide scalar
   // loads, no guards); ND = 0: guarded by the runtime n_dist (<= 10)
@@ -195,15 +173,13 @@ __device__ __forceinline__ double openness_angle_s(const WinDevR& W, int i, int 
     float ext = __builtin_nanf("");
 #pragma unroll
     for (int k = 0; k < NU; k++) ext = NEG ? fminf(ext, q[k]) : fmaxf(ext, q[k]);
-    if (isnan(ext)) S.missing++;
-    else S.add<NEG>(ext);
-    if ((d & 3) == 3) S.rescale();
+    if (!isnan(ext)) S.add<NEG>(ext);
   }
-  return S.mean(T);
+  return S.mean();
 }
 
 template <int ND, bool CHECK, bool OFF32 = false>
-__device__ __forceinline__ double openness_angle_u(const WinDevR& W, int i, int j, float z,
+__device__ __forceinline__ float openness_angle_u(const WinDevR& W, int i, int j, float z,
                                                   const OpenTab& T) {
   return T.negative ? openness_angle_s<ND, CHECK, OFF32, true>(W, i, j, z, T)
                     : openness_angle_s<ND, CHECK, OFF32, false>(W, i, j, z, T);
@@ -217,7 +193,7 @@ __device__ __forceinline__ bool open_off32(const WinDevR& W, const OpenTab& T) {
 
 // Mean angle at (i, j): the unrolled variant when the table allows it.
 // interior: the caller knows every sample of (i, j) lies inside the window.
-__device__ __forceinline__ double openness_angle_at(const WinDevR& W, int i, int j, float z,
+__device__ __forceinline__ float openness_angle_at(const WinDevR& W, int i, int j, float z,
                                                    const OpenTab& T, bool interior) {
   if (T.n_dist == OPEN_UNROLL) {
     if (!interior) return openness_angle_u<OPEN_UNROLL, true>(W, i, j, z, T);
@@ -236,9 +212,10 @@ __device__ __forceinline__ bool openness_interior(const WinDevR& W, const OpenTa
 }
 
 // display value (op / (pi/2), clipped, gamma) or, with T.raw, the angle in degrees
-__device__ __forceinline__ float openness_value(const OpenTab& T, double angle) {
-  if (T.raw) return (float)(angle * (180.0 / M_PI));
-  return gamma_pow(fmin(fmax(angle * (2.0 / M_PI), 0.0), 1.0));
+__device__ __forceinline__ float openness_value(const OpenTab& T, float angle) {
+  if (T.raw) return (float)((double)angle * (180.0 / M_PI));
+  const float op = fminf(fmaxf(angle / 1.57079637f, 0.0f), 1.0f);
+  return powf(op, (float)(1.0 / 2.2));
 }
 
 // The device ray table of an fsg_openness_params (offsets and f32(1/phys)).
@@ -253,7 +230,6 @@ inline int openness_table(const fsg_openness_params* p, OpenTab& T, const char* 
   T.n_dist = p->n_dist;
   T.negative = p->openness_type != 0;
   T.raw = p->raw_degrees != 0;
-  T.inv_dirs = 1.0 / std::max(1, p->n_dirs);
   for (int e = 0; e < p->n_dirs * p->n_dist; e++) {
     const fsg_ray_sample& s = p->samples[e];
     if (s.skip || (s.dx == 0 && s.dy == 0)) {
