@@ -100,7 +100,7 @@ __device__ __forceinline__ void openness_item(const OpenTileD& O, const OpenTab&
 
 template <int NR, int KINDS>
 __device__ __forceinline__ void batch_drain(const BatchDev& B) {
-  extern __shared__ float lds[];
+  extern __shared__ __attribute__((aligned(16))) float lds[];
   __shared__ int s_item;
   const int n_stencil = B.n_st_items;
   const int total = B.n_usm_items + n_stencil + B.n_op_items;

@@ -103,7 +103,7 @@ __global__ void k_ovr_avg(const T* __restrict__ src, int64_t lds, int h, int w,
 template <typename T>
 __global__ void k_tile_encode(const T* __restrict__ lvl, int64_t ld, int h, int w, int block,
                               int ntx, int t0, int predictor, T pad, uint8_t* __restrict__ out) {
-  extern __shared__ uint8_t rowb[];
+  extern __shared__ __attribute__((aligned(16))) uint8_t rowb[];
   const int t = t0 + blockIdx.y, r = blockIdx.x;
   const int ty = t / ntx, tx = t % ntx;
   const int y = ty * block + r;
@@ -154,7 +154,7 @@ __global__ void __launch_bounds__(256) k_tile_decode(const uint8_t* __restrict__
                                                      int tw, int th, int predictor, int r0,
                                                      int c0, int wh, int ww,
                                                      T* __restrict__ out, int64_t ldo) {
-  extern __shared__ uint8_t smem[];
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   constexpr int B = sizeof(T);
   const int r = blockIdx.x;
   const DecTile dt = tiles[blockIdx.y];

@@ -417,6 +417,7 @@ __device__ __forceinline__ void stencil_tile_block_v(const StencilTile& S, int b
       if (__syncthreads_or(hole) && __syncthreads_or(valid)) {
         constexpr int FW = ST_TW + 2 * ST_HALO + 8;             // column sums of a row
         constexpr int NAN_ROWS = (2 * ST_PH * ST_PW) / (2 * FW);  // rows that fit
+        static_assert(ST_ROWS * ST_LT % 2 == 0, "the sums are float2 from Pt on");
         float2* sums = (float2*)Pt;
         for (int b0 = 0; b0 < nr; b0 += NAN_ROWS) {
           const int n = min(NAN_ROWS, nr - b0);

@@ -655,7 +655,7 @@ template <int NR, bool NANAW, int K, bool GAUSS>
 __global__ void __launch_bounds__(256) k_usm_main(UsmArgs A) {
   constexpr int KS = 8;           // rows per batch of column loads
   constexpr int NRA = NR > 0 ? NR : 1;
-  extern __shared__ float lds[];
+  extern __shared__ __attribute__((aligned(16))) float lds[];
   const int NC = A.SW + 2 * A.R;
   const int LDC = NC + 1;         // padded LDS row stride
   float* Vs = lds;                                   // [NR][K][LDC] axis-0 means
@@ -962,7 +962,7 @@ static int dispatch_usm(const UsmArgs& A, bool nanaw, int n_blocks, hipStream_t 
 // the region land on one XCD (L2).
 template <int NR, bool NANAW>
 __global__ void __launch_bounds__(256) k_usm_fast(UsmArgs A, int n_tiles, int per_xcd) {
-  extern __shared__ float lds[];
+  extern __shared__ __attribute__((aligned(16))) float lds[];
   const int b = blockIdx.x;
   const int tile = (b & 7) * per_xcd + (b >> 3);
   if (tile >= n_tiles) return;

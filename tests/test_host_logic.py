@@ -262,3 +262,20 @@ def test_ray_sample_arrays_equal_the_tables(n, dist, px, sx, sy):
         assert bool(g["skip"]) == (w is None)
         if w is not None:
             assert (int(g["dx"]), int(g["dy"]), float(g["phys"]), float(g["dist_factor"])) == w
+
+
+def test_dynamic_lds_is_declared_at_16_bytes():
+    """Every kernel carves float2, double or 16-byte entries out of its dynamic LDS at
+    offsets of whole 8 or 16 bytes, so the array itself starts at 16: without the
+    attribute it starts behind the static LDS at its element type's alignment."""
+    import glob
+    import os
+    import re
+    csrc = os.path.join(os.path.dirname(__file__), "..", "fujishadergpu_amd", "csrc")
+    n = 0
+    for path in sorted(glob.glob(os.path.join(csrc, "*.h*"))):
+        with open(path, encoding="utf-8") as fh:
+            for decl in re.findall(r"extern __shared__[^;]*;", fh.read()):
+                assert "__attribute__((aligned(16)))" in decl, f"{os.path.basename(path)}: {decl}"
+                n += 1
+    assert n >= 9
