@@ -161,11 +161,16 @@ def ray_samples(ox: np.ndarray, oy: np.ndarray, sx: float, sy: float,
     return out
 
 
+def _is_records(table) -> bool:
+    """Whether a table is a record array; an array of plain numbers is a sequence."""
+    return isinstance(table, np.ndarray) and table.dtype.names is not None
+
+
 def openness_params(table, openness_type: str, raw_degrees: bool = False):
     """(params, keep-alive array) for a ray table: a (directions, distances)
-    RAY_SAMPLE array, or a list over directions of lists over distances of
-    (ox, oy, phys)|None."""
-    if isinstance(table, np.ndarray):
+    RAY_SAMPLE array, or a sequence over directions of sequences over distances
+    of (ox, oy, phys)|None."""
+    if _is_records(table):
         arr = np.ascontiguousarray(table, dtype=RAY_SAMPLE)
         return N.fsg_openness_params(
             0 if openness_type == "positive" else 1, arr.shape[0], arr.shape[1],
@@ -267,19 +272,24 @@ def openness_judge(win_t, approx: torch.Tensor, *, tile_h: int, tile_w: int, sam
     return out
 
 
-def ambient_occlusion(win_t, reg, *, table, intensity: float, pad_d: int,
-                      out: N.fsg_output) -> None:
-    """table: an AO_SAMPLE array, or a list of (dx, dy, phys, dist_factor)|None, in
-    reference order."""
-    if isinstance(table, np.ndarray):
+def ao_params(table, intensity: float, pad_d: int):
+    """(params, keep-alive array) for a sample table: an AO_SAMPLE array, or a sequence
+    of (dx, dy, phys, dist_factor)|None, in reference order."""
+    if _is_records(table):
         arr = np.ascontiguousarray(table, dtype=AO_SAMPLE)
     else:
         arr = np.zeros(len(table), dtype=AO_SAMPLE)
         for i, entry in enumerate(table):
             arr[i] = (0, 0, 1, 0, 0.0, 0.0) if entry is None else \
                 (int(entry[0]), int(entry[1]), 0, 0, float(entry[2]), float(entry[3]))
-    p = N.fsg_ao_params(len(arr), int(pad_d), float(intensity),
-                        C.cast(arr.ctypes.data, C.POINTER(N.fsg_ao_sample)))
+    return N.fsg_ao_params(len(arr), int(pad_d), float(intensity),
+                           C.cast(arr.ctypes.data, C.POINTER(N.fsg_ao_sample))), arr
+
+
+def ambient_occlusion(win_t, reg, *, table, intensity: float, pad_d: int,
+                      out: N.fsg_output) -> None:
+    """table: as ao_params takes it."""
+    p, _arr = ao_params(table, intensity, pad_d)
     w = window(win_t)
     L = _lib()
     nbytes = L.fsg_ambient_occlusion_workspace_size(C.byref(w), C.byref(reg))

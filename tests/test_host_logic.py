@@ -279,3 +279,24 @@ def test_dynamic_lds_is_declared_at_16_bytes():
                 assert "__attribute__((aligned(16)))" in decl, f"{os.path.basename(path)}: {decl}"
                 n += 1
     assert n >= 9
+
+
+def test_ray_tables_given_as_plain_number_arrays():
+    """A table as an array of plain numbers, (directions, distances, 3) or (samples, 4), is
+    read entry by entry as the list of its rows is."""
+    import numpy as np
+    from fujishadergpu_amd import ops
+    from fujishadergpu_amd.algorithms import ao_table, openness_table
+    table = openness_table(6, 20, 5.0)
+    got, want = (ops.openness_params(t, "negative", True)[0] for t in (np.array(table), table))
+    assert (got.n_dirs, got.n_dist) == (want.n_dirs, want.n_dist) == (6, 10)
+    for e in range(60):
+        g, w = got.samples[e], want.samples[e]
+        assert (g.dx, g.dy, g.skip, g.phys) == (w.dx, w.dy, w.skip, w.phys)
+    ring = ao_table(5, 12.0, 5.0)
+    got, want = (ops.ao_params(t, 1.0, 12)[0] for t in (np.array(ring), ring))
+    assert got.n_samples == want.n_samples == 20
+    for e in range(20):
+        g, w = got.samples[e], want.samples[e]
+        assert (g.dx, g.dy, g.skip, g.phys, g.dist_factor) == \
+            (w.dx, w.dy, w.skip, w.phys, w.dist_factor)
