@@ -50,14 +50,20 @@ def valid_bbox_begin(raster: torch.Tensor):
     H, W = raster.shape
     cov = max(1, max(W, H) // 512)
     oh, ow = max(1, H // cov), max(1, W // cov)
-    if not raster.is_cuda:
-        ri, ci = (torch.clamp(((torch.arange(n, dtype=torch.float64) + 0.5) * (full / n))
-                              .floor().long(), max=full - 1) for n, full in ((oh, H), (ow, W)))
-        return raster.index_select(0, ri).index_select(1, ci), None, cov, H, W
-    # the same positions, in one launch
-    ov = torch.empty((oh, ow), dtype=torch.float32, device=raster.device)
-    win = ops.window(raster)
-    N.check(N.lib().fsg_prepare_sample(C.byref(win), oh, ow, ov.data_ptr(), ow, ops._stream()))
+    if (raster.is_cuda and raster.dtype == torch.float32 and raster.stride(1) == 1 and
+            raster.stride(0) >= W):
+        # the same positions as below, in one launch
+        ov = torch.empty((oh, ow), dtype=torch.float32, device=raster.device)
+        win = ops.window(raster)
+        N.check(N.lib().fsg_prepare_sample(C.byref(win), oh, ow, ov.data_ptr(), ow,
+                                           ops._stream()))
+    else:
+        ri, ci = (torch.clamp(((torch.arange(n, device=raster.device, dtype=torch.float64) + 0.5)
+                               * (full / n)).floor().long(), max=full - 1)
+                  for n, full in ((oh, H), (ow, W)))
+        ov = raster.index_select(0, ri).index_select(1, ci)
+        if not raster.is_cuda:
+            return ov, None, cov, H, W
     host = torch.empty((oh, ow), dtype=raster.dtype, pin_memory=True)
     host.copy_(ov, non_blocking=True)
     ev = torch.cuda.Event()

@@ -857,3 +857,25 @@ def test_nan_aware_box_bands_match_the_oracle(cuda, h, w, radii):
     for g, r in zip(got, radii):
         want, _ = ref.handle_nan_with_uniform(dem.numpy(), size=2 * r + 1, mode="reflect")
         assert np.abs(g - want).max() <= 3e-4
+
+
+@pytest.mark.parametrize("kind", ["float32", "float64", "int32", "transposed", "column_step",
+                                  "one_row_repeated"])
+def test_valid_bbox_of_any_raster_on_the_gpu(cuda, kind):
+    """The overview's bounding box for rasters that are no float32 row windows too: the
+    box that the same raster gives on the CPU."""
+    from fujishadergpu_amd.stats import valid_bbox
+    a = torch.full((1300, 1700), float("nan"))
+    a[310:905, 120:1411] = 7.0
+    if kind == "int32":
+        a = torch.nan_to_num(a).to(torch.int32)
+    elif kind == "float64":
+        a = a.double()
+    g = a.to(cuda)
+    if kind == "transposed":
+        a, g = a.t(), g.t()
+    elif kind == "column_step":
+        a, g = a[:, ::2], g[:, ::2]
+    elif kind == "one_row_repeated":
+        a, g = a[400:401].expand(900, 1700), g[400:401].expand(900, 1700)
+    assert valid_bbox(g) == valid_bbox(a)
