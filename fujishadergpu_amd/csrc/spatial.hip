@@ -360,7 +360,7 @@ __global__ __launch_bounds__(256, 2) void k_gauss_nan_cols(const float* __restri
 }
 
 // The copies and interpolations below give a wave 256 columns, four per lane 64
-// apart (each access 256 contiguous bytes), and ROW_WALK rows of them: what a
+// apart (each access 256 contiguous bytes), and `walk` rows of them: what a
 // column or a pair of source rows determines is computed once per walk.  One
 // pixel per thread redid it (and, for the interpolations, eight float64
 // conversions and two lerps) for every output.
@@ -369,22 +369,30 @@ constexpr int ROW_WALK = 16;
 struct Strip {
   int x, y0, rows;   // this lane's first column, the wave's rows
 };
-__device__ __forceinline__ Strip row_strip(int h) {
+__device__ __forceinline__ Strip row_strip(int h, int walk) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   Strip p;
   p.x = blockIdx.x * 256 + (threadIdx.x & 63);
-  p.y0 = (blockIdx.y * 4 + wave) * ROW_WALK;
-  p.rows = min(ROW_WALK, h - p.y0);
+  p.y0 = (blockIdx.y * 4 + wave) * walk;
+  p.rows = min(walk, h - p.y0);
   return p;
 }
-static dim3 strip_grid(int w, int h) {
-  return dim3((unsigned)((w + 255) / 256), (unsigned)((h + 4 * ROW_WALK - 1) / (4 * ROW_WALK)));
+// The rows of a wave: ROW_WALK, more where the grid's 65535 block rows would not
+// cover the extent.
+static int strip_walk(int h) {
+  constexpr int64_t max_rows = 4 * 65535;
+  return (int)std::max<int64_t>(ROW_WALK, (h + max_rows - 1) / max_rows);
+}
+static dim3 strip_grid(int w, int h, int walk) {
+  const int64_t rows = 4 * (int64_t)walk;
+  return dim3((unsigned)(((int64_t)w + 255) / 256), (unsigned)((h + rows - 1) / rows));
 }
 
 // 4384^2 padded by 65 or 257: 116 us a launch in an 8192^2 job, now 48.
-__global__ void __launch_bounds__(256) k_pad_sym(PadSrc S, float* __restrict__ out, int64_t ldo) {
+__global__ void __launch_bounds__(256) k_pad_sym(PadSrc S, float* __restrict__ out, int64_t ldo,
+                                                 int walk) {
   const int hp = S.h + 2 * S.pad, wp = S.w + 2 * S.pad;
-  const Strip p = row_strip(hp);
+  const Strip p = row_strip(hp, walk);
   int col[4];
 #pragma unroll
   for (int m = 0; m < 4; m++) col[m] = sym(min(p.x + 64 * m, wp - 1) - S.pad, S.w);
@@ -416,8 +424,8 @@ __global__ void __launch_bounds__(256) k_pad_sym(PadSrc S, float* __restrict__ o
 // 1129^2 to 4516^2: 114 us, now 39.
 __global__ void __launch_bounds__(256)
 k_upsample_shape(const float* __restrict__ src, int64_t lds, int hs, int ws, int zh, int zw,
-                 float* __restrict__ out, int64_t ldo, int h, int w) {
-  const Strip p = row_strip(h);
+                 float* __restrict__ out, int64_t ldo, int h, int w, int walk) {
+  const Strip p = row_strip(h, walk);
   if (p.rows <= 0) return;
   const double zx = zw > 1 ? (double)(ws - 1) / (double)(zw - 1) : 0.0;
   const double zy = zh > 1 ? (double)(hs - 1) / (double)(zh - 1) : 0.0;
@@ -473,8 +481,8 @@ k_upsample_shape(const float* __restrict__ src, int64_t lds, int hs, int ws, int
 __global__ void __launch_bounds__(256)
 k_sample_coarse(const float* __restrict__ coarse, int64_t ldc, int hc, int wc, int r0, int c0,
                 float fy, float fx, const float* __restrict__ win, int64_t ldw,
-                float* __restrict__ out, int64_t ldo, int h, int w) {
-  const Strip p = row_strip(h);
+                float* __restrict__ out, int64_t ldo, int h, int w, int walk) {
+  const Strip p = row_strip(h, walk);
   if (p.rows <= 0) return;
   int x0[4], x1[4];
   double tx[4];
@@ -654,7 +662,9 @@ extern "C" int fsg_pad_symmetric(const fsg_window* src, int32_t pad, float* out,
     return fail(FSG_E_INVALID, "fsg_pad_symmetric: bad arguments (pad must be <= the window)");
   const int hp = src->h + 2 * pad, wp = src->w + 2 * pad;
   PadSrc S{src->data, src->ld, src->h, src->w, pad};
-  hipLaunchKernelGGL(k_pad_sym, strip_grid(wp, hp), dim3(256), 0, as_stream(stream), S, out, ldo);
+  const int walk = strip_walk(hp);
+  hipLaunchKernelGGL(k_pad_sym, strip_grid(wp, hp, walk), dim3(256), 0, as_stream(stream), S, out,
+                     ldo, walk);
   FSG_CHECK_LAUNCH("k_pad_sym");
   return FSG_OK;
 }
@@ -694,8 +704,9 @@ extern "C" int fsg_upsample_to_shape(const float* src, int64_t lds, int32_t hs, 
   // scipy zoom output shape: round(n_in * (N / n_in))
   const int zh = (int)std::nearbyint((double)hs * ((double)h / (double)hs));
   const int zw = (int)std::nearbyint((double)ws * ((double)w / (double)ws));
-  hipLaunchKernelGGL(k_upsample_shape, strip_grid(w, h), dim3(256), 0, as_stream(stream), src, lds,
-                     hs, ws, std::max(1, zh), std::max(1, zw), out, ldo, h, w);
+  const int walk = strip_walk(h);
+  hipLaunchKernelGGL(k_upsample_shape, strip_grid(w, h, walk), dim3(256), 0, as_stream(stream), src,
+                     lds, hs, ws, std::max(1, zh), std::max(1, zw), out, ldo, h, w, walk);
   FSG_CHECK_LAUNCH("k_upsample_shape");
   return FSG_OK;
 }
@@ -708,8 +719,9 @@ extern "C" int fsg_sample_coarse(const float* coarse, int64_t ldc, int32_t hc, i
       ldc < wc || ldo < w || (nan_src && ld_nan < w))
     return fail(FSG_E_INVALID, "fsg_sample_coarse: bad arguments");
   const float fy = (float)((double)hc / (double)full_h), fx = (float)((double)wc / (double)full_w);
-  hipLaunchKernelGGL(k_sample_coarse, strip_grid(w, h), dim3(256), 0, as_stream(stream), coarse, ldc,
-                     hc, wc, r0, c0, fy, fx, nan_src, ld_nan, out, ldo, h, w);
+  const int walk = strip_walk(h);
+  hipLaunchKernelGGL(k_sample_coarse, strip_grid(w, h, walk), dim3(256), 0, as_stream(stream),
+                     coarse, ldc, hc, wc, r0, c0, fy, fx, nan_src, ld_nan, out, ldo, h, w, walk);
   FSG_CHECK_LAUNCH("k_sample_coarse");
   return FSG_OK;
 }

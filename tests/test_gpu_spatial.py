@@ -378,3 +378,18 @@ def test_combine_at_ragged_extents_and_offsets(cuda, dtype, agg, h, w, off):
     got = big.cpu().numpy()
     assert np.array_equal(got[:, off:off + w], exp, equal_nan=dtype == "float32")
     assert not got[:, :off].any() and not got[:, off + w:].any()
+
+
+def test_strip_kernels_cover_more_rows_than_the_grid_holds(cuda):
+    """One row past 65536 blocks of 64 rows, where the walks have to be longer."""
+    from fujishadergpu_amd import spatial
+    h = 65536 * 64 + 1
+    src = torch.arange(h, dtype=torch.float32, device=cuda).view(h, 1)
+    padded = spatial.pad_symmetric(src, 1)
+    assert torch.equal(padded[1:-1, 1], src[:, 0])
+    assert padded[0, 0] == src[0, 0] and padded[-1, 2] == src[-1, 0]
+    flat = torch.full((3, 1), 5.0, device=cuda)
+    assert bool((spatial.upsample_to_shape(flat, h, 1) == 5.0).all())
+    out = torch.zeros((h, 1), device=cuda)
+    spatial._sample(flat, 0, 0, h, 1, src, out)
+    assert bool((out == 5.0).all())
