@@ -377,18 +377,24 @@ __device__ __forceinline__ Strip row_strip(int h, int walk) {
   p.rows = min(walk, h - p.y0);
   return p;
 }
-// The rows of a wave: ROW_WALK, more where the grid's 65535 block rows would not
-// cover the extent.
-static int strip_walk(int h) {
+// The rows of a wave: ROW_WALK, fewer where that would leave the launch less than
+// WALK_WAVES waves (a walk is one wave's chain: 1024^2 overview samples 13.3 us in
+// walks of 16 rows, 7.4 of 1, 7.2 one pixel per thread; 2048^2 15.5, 9.0 of 4,
+// 11.9; upsampling 2048^2 9.3 of 4 rows, 10.9 of 2, 13.7 of 1), more where the
+// grid's 65535 block rows would not cover the extent.
+constexpr int64_t WALK_WAVES = 4096;
+static int strip_walk(int w, int h) {
   constexpr int64_t max_rows = 4 * 65535;
-  return (int)std::max<int64_t>(ROW_WALK, (h + max_rows - 1) / max_rows);
+  const int64_t rows = ((int64_t)w + 255) / 256 * h / WALK_WAVES;
+  return (int)std::max(std::min<int64_t>(ROW_WALK, std::max<int64_t>(1, rows)),
+                       (h + max_rows - 1) / max_rows);
 }
 static dim3 strip_grid(int w, int h, int walk) {
   const int64_t rows = 4 * (int64_t)walk;
   return dim3((unsigned)(((int64_t)w + 255) / 256), (unsigned)((h + rows - 1) / rows));
 }
 
-// 4384^2 padded by 65 or 257: 116 us a launch in an 8192^2 job, now 48.
+// 4096^2 padded by 32: 31 us, now 22.
 __global__ void __launch_bounds__(256) k_pad_sym(PadSrc S, float* __restrict__ out, int64_t ldo,
                                                  int walk) {
   const int hp = S.h + 2 * S.pad, wp = S.w + 2 * S.pad;
@@ -421,7 +427,7 @@ __global__ void __launch_bounds__(256) k_pad_sym(PadSrc S, float* __restrict__ o
 // valid, num / max(den, 1e-6) where den > 1e-3 else NaN; the zoom output
 // shape round(n_in * (N / n_in)) is edge-padded (or cropped) to N.  A
 // NaN-free source gives den = 1 and the plain zoom bit for bit.
-// 1129^2 to 4516^2: 114 us, now 39.
+// 1024^2 to 4096^2: 65 us, now 22.
 __global__ void __launch_bounds__(256)
 k_upsample_shape(const float* __restrict__ src, int64_t lds, int hs, int ws, int zh, int zw,
                  float* __restrict__ out, int64_t ldo, int h, int w, int walk) {
@@ -477,7 +483,7 @@ k_upsample_shape(const float* __restrict__ src, int64_t lds, int hs, int ws, int
 // _bilinear_sample_coarse (_nan_utils.py:255-281): map_coordinates order 1,
 // mode 'nearest', at float32 coordinates (g + 0.5) * f32(n_c / N) - 0.5 of the
 // window's raster rows r0 + i and columns c0 + j; NaN where the window is NaN.
-// 2048^2 overview, 4096^2 window: 96 us, now 48.
+// 1024^2 overview, 4096^2 window: 42 us, now 30.
 __global__ void __launch_bounds__(256)
 k_sample_coarse(const float* __restrict__ coarse, int64_t ldc, int hc, int wc, int r0, int c0,
                 float fy, float fx, const float* __restrict__ win, int64_t ldw,
@@ -662,7 +668,7 @@ extern "C" int fsg_pad_symmetric(const fsg_window* src, int32_t pad, float* out,
     return fail(FSG_E_INVALID, "fsg_pad_symmetric: bad arguments (pad must be <= the window)");
   const int hp = src->h + 2 * pad, wp = src->w + 2 * pad;
   PadSrc S{src->data, src->ld, src->h, src->w, pad};
-  const int walk = strip_walk(hp);
+  const int walk = strip_walk(wp, hp);
   hipLaunchKernelGGL(k_pad_sym, strip_grid(wp, hp, walk), dim3(256), 0, as_stream(stream), S, out,
                      ldo, walk);
   FSG_CHECK_LAUNCH("k_pad_sym");
@@ -704,7 +710,7 @@ extern "C" int fsg_upsample_to_shape(const float* src, int64_t lds, int32_t hs, 
   // scipy zoom output shape: round(n_in * (N / n_in))
   const int zh = (int)std::nearbyint((double)hs * ((double)h / (double)hs));
   const int zw = (int)std::nearbyint((double)ws * ((double)w / (double)ws));
-  const int walk = strip_walk(h);
+  const int walk = strip_walk(w, h);
   hipLaunchKernelGGL(k_upsample_shape, strip_grid(w, h, walk), dim3(256), 0, as_stream(stream), src,
                      lds, hs, ws, std::max(1, zh), std::max(1, zw), out, ldo, h, w, walk);
   FSG_CHECK_LAUNCH("k_upsample_shape");
@@ -719,7 +725,7 @@ extern "C" int fsg_sample_coarse(const float* coarse, int64_t ldc, int32_t hc, i
       ldc < wc || ldo < w || (nan_src && ld_nan < w))
     return fail(FSG_E_INVALID, "fsg_sample_coarse: bad arguments");
   const float fy = (float)((double)hc / (double)full_h), fx = (float)((double)wc / (double)full_w);
-  const int walk = strip_walk(h);
+  const int walk = strip_walk(w, h);
   hipLaunchKernelGGL(k_sample_coarse, strip_grid(w, h, walk), dim3(256), 0, as_stream(stream),
                      coarse, ldc, hc, wc, r0, c0, fy, fx, nan_src, ld_nan, out, ldo, h, w, walk);
   FSG_CHECK_LAUNCH("k_sample_coarse");

@@ -315,7 +315,9 @@ def test_gaussian_band_products_against_float64(cuda, h, w, pad, sigma, special)
 
 
 @pytest.mark.parametrize("h,w,hs,ws", [(1, 1, 1, 1), (17, 255, 5, 64), (64, 257, 16, 65),
-                                       (145, 600, 10, 38), (33, 130, 33, 130)])
+                                       (145, 600, 10, 38), (33, 130, 33, 130),
+                                       # walks of 2 and of 16 rows (one row above)
+                                       (2049, 1030, 130, 65), (3900, 4355, 60, 50)])
 @pytest.mark.parametrize("nan", [False, True])
 def test_strip_kernels_at_ragged_extents(cuda, h, w, hs, ws, nan):
     """Upsampling, the overview sample and the symmetric pad over partial strips and walks,
