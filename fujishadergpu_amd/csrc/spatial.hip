@@ -359,6 +359,201 @@ __global__ __launch_bounds__(256, 2) void k_gauss_nan_cols(const float* __restri
       }
 }
 
+// ---------------------------------------- the same passes on the vector units
+//
+// Small extents: the products' tiles of 128 x 64 leave most CUs idle there, and a
+// tile's chain (twice the staging, a band and marks to read) is longer.  64 x 64
+// tiles; each of the 4 waves of a block owns GN_M consecutive outputs along the
+// filter axis for 64 lines across it, so one sample loaded from LDS into a
+// register serves GN_M outputs: the pair (x[-d], x[+d]) of output m at distance d
+// is x[m - d], x[m + d], and a block of GN_M distances reads two register windows
+// of 2 GN_M - 1 samples that slide by GN_M per block.  Sums in scipy's symmetric
+// order, as gn_slow's.
+constexpr int GN_M = 16;   // outputs per lane along the filter axis (4 waves x 16 = 64)
+
+// acc[m] = sum_k g[|k|] v(s[(m + k) ST]), k in [-r, r], in the order above.
+// s points at the lane's first output; the LDS line holds r samples before
+// it and r + GN_M - 1 after it.
+template <int MODE, int ST>
+__device__ __forceinline__ void gn_line(const float* s, const GaussW& G, double (&acc)[GN_M]) {
+  const double g0 = G.g[0];
+#pragma unroll
+  for (int m = 0; m < GN_M; m++) acc[m] = gn_val<MODE>(s[m * ST]) * g0;
+  int d = G.r;
+  for (; d % GN_M != 0; d--) {   // the top r mod GN_M distances one at a time
+    const double g = G.g[d];
+#pragma unroll
+    for (int m = 0; m < GN_M; m++)
+      acc[m] = acc[m] + (gn_val<MODE>(s[(m - d) * ST]) + gn_val<MODE>(s[(m + d) * ST])) * g;
+  }
+  if (d == 0) return;
+  // distances d .. d - GN_M + 1: L[k] = x[k - d], R[k] = x[k + d - GN_M + 1]
+  double L[2 * GN_M - 1], R[2 * GN_M - 1];
+#pragma unroll
+  for (int k = 0; k < 2 * GN_M - 1; k++) {
+    L[k] = gn_val<MODE>(s[(k - d) * ST]);
+    R[k] = gn_val<MODE>(s[(k + d - (GN_M - 1)) * ST]);
+  }
+  for (;;) {
+#pragma unroll
+    for (int dd = 0; dd < GN_M; dd++) {
+      const double g = G.g[d - dd];
+#pragma unroll
+      for (int m = 0; m < GN_M; m++) acc[m] = acc[m] + (L[m + dd] + R[m - dd + GN_M - 1]) * g;
+    }
+    d -= GN_M;
+    if (d == 0) break;
+#pragma unroll
+    for (int k = 0; k < GN_M - 1; k++) L[k] = L[k + GN_M];
+#pragma unroll
+    for (int k = GN_M - 1; k < 2 * GN_M - 1; k++) L[k] = gn_val<MODE>(s[(k - d) * ST]);
+#pragma unroll
+    for (int k = 2 * GN_M - 2; k >= GN_M; k--) R[k] = R[k - GN_M];
+#pragma unroll
+    for (int k = 0; k < GN_M; k++) R[k] = gn_val<MODE>(s[(k + d - (GN_M - 1)) * ST]);
+  }
+}
+
+// Pass 0: tv and tw as k_gauss_nan_rows forms them, tw written everywhere (f32(wsum)
+// in a tile without NaN).  LDS: (64 + 2r) rows x 64 columns.
+__global__ __launch_bounds__(256, 2) void k_gauss_tap_rows(PadSrc S, GaussW G,
+                                                           float* __restrict__ tv,
+                                                           float* __restrict__ tw, int64_t ldt,
+                                                           float wconst) {
+  extern __shared__ __attribute__((aligned(16))) float gl[];
+  const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
+  const int hp = S.h + 2 * S.pad, wp = S.w + 2 * S.pad;
+  const int tx0 = blockIdx.x * GN_T, ty0 = blockIdx.y * GN_T;
+  const int nrow = GN_T + 2 * G.r;
+  const int pc = min(tx0 + lane, wp - 1);
+  bool nan = false;
+  // staging in batches of 8 rows per wave (8 loads in flight per lane)
+  for (int i0 = q; i0 < nrow; i0 += 32) {
+    float v[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      const int i = i0 + 4 * u;
+      v[u] = i < nrow ? S.at(ty0 - G.r + i, pc) : 0.0f;
+    }
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+      const int i = i0 + 4 * u;
+      if (i < nrow) {
+        gl[i * GN_T + lane] = v[u];
+        nan |= isnan(v[u]);
+      }
+    }
+  }
+  const bool any_nan = __syncthreads_or(nan);
+  const float* s = gl + (q * GN_M + G.r) * GN_T + lane;
+  const int x = tx0 + lane;
+  const int y0 = ty0 + q * GN_M;
+  const int nm = x < wp ? min(GN_M, hp - y0) : 0;   // rows this lane stores
+  double acc[GN_M];
+  if (any_nan) gn_line<1, GN_T>(s, G, acc);
+  else gn_line<0, GN_T>(s, G, acc);
+#pragma unroll
+  for (int m = 0; m < GN_M; m++)
+    if (m < nm) tv[(int64_t)(y0 + m) * ldt + x] = (float)acc[m];
+  if (!any_nan) {
+#pragma unroll
+    for (int m = 0; m < GN_M; m++)
+      if (m < nm) tw[(int64_t)(y0 + m) * ldt + x] = wconst;
+    return;
+  }
+  gn_line<2, GN_T>(s, G, acc);
+#pragma unroll
+  for (int m = 0; m < GN_M; m++)
+    if (m < nm) tw[(int64_t)(y0 + m) * ldt + x] = (float)acc[m];
+}
+
+// Pass 1.  A tile whose tw span is all f32(wsum) divides by the constant wdiv.  LDS:
+// 64 rows x (64 + 2r + 1) columns (odd pitch: lanes walk rows without bank
+// conflicts), reused for tw, tv and the transposed output tile.
+__global__ __launch_bounds__(256, 2) void k_gauss_tap_cols(const float* __restrict__ tv,
+                                                        const float* __restrict__ tw, int64_t ldt,
+                                                        int hp, int wp, GaussW G,
+                                                        float* __restrict__ out, int64_t ldo,
+                                                        float wconst, float wdiv) {
+  extern __shared__ __attribute__((aligned(16))) float gl[];
+  const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
+  const int tx0 = blockIdx.x * GN_T, ty0 = blockIdx.y * GN_T;
+  const int ncol = GN_T + 2 * G.r, P = ncol + 1;
+  // staging: column chunks of 64, each in batches of 8 rows per wave (8 loads in flight)
+  auto stage = [&](const float* src) {
+    bool off = false;
+    for (int c = 0; c < ncol; c += 64) {
+      const int j = c + lane;
+      const bool jok = j < ncol;
+      const int col = min(max(tx0 - G.r + j, 0), wp - 1);
+#pragma unroll
+      for (int k0 = 0; k0 < GN_T / 4; k0 += 8) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+          const int i = q + 4 * (k0 + u);
+          v[u] = jok ? src[(int64_t)min(ty0 + i, hp - 1) * ldt + col] : 0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+          const int i = q + 4 * (k0 + u);
+          if (jok) {
+            gl[i * P + j] = v[u];
+            off |= __float_as_uint(v[u]) != __float_as_uint(wconst);
+          }
+        }
+      }
+    }
+    return off;
+  };
+  const float* s = gl + lane * P + q * GN_M + G.r;
+  double acc[GN_M];
+  float fw[GN_M], fo[GN_M];
+  const bool varied = __syncthreads_or(stage(tw));
+  if (varied) {
+    gn_line<0, 1>(s, G, acc);
+#pragma unroll
+    for (int m = 0; m < GN_M; m++) fw[m] = (float)acc[m];
+  } else {
+#pragma unroll
+    for (int m = 0; m < GN_M; m++) fw[m] = wdiv;
+  }
+  __syncthreads();
+  stage(tv);
+  __syncthreads();
+  gn_line<0, 1>(s, G, acc);
+#pragma unroll
+  for (int m = 0; m < GN_M; m++) {
+    const float v = (float)acc[m];
+    fo[m] = fw[m] > 0.0f ? v / fw[m] : 0.0f;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < GN_M; m++) gl[lane * (GN_T + 1) + q * GN_M + m] = fo[m];
+  __syncthreads();
+  const int x = tx0 + lane;
+  if (x >= wp) return;
+  for (int i = q; i < GN_T; i += 4) {
+    const int y = ty0 + i;
+    if (y < hp) out[(int64_t)y * ldo + x] = gl[i * (GN_T + 1) + lane];
+  }
+}
+
+// The extents that take the vector units, by their 64 x 64 tiles.  Both passes in us,
+// vector / products, without NaN and with 1 % of discs: r = 2 at 1024 tiles 40 / 42
+// and 42 / 48, at 1444 53 / 49 and 54 / 55; r = 8 (its distances all one at a time)
+// at 529 39 / 39 and 40 / 44, at 1024 49 / 44 and 58 / 50; r = 16 at 729 42 / 43 and
+// 47 / 54, at 1089 60 / 57 and 63 / 71, at 1444 67 / 57 and 71 / 69; r = 32 at 729
+// 53 / 51 and 62 / 69, at 1024 63 / 56 and 77 / 74; r = 64 at 529 75 / 69 and 82 / 97,
+// at 729 77 / 68 and 108 / 99; r = 160 (one block a CU) at 256 76 / 81 and 111 / 130,
+// at 289 132 / 80 and 170 / 131.
+static bool gauss_vector(int hp, int wp, int r) {
+  const int64_t tiles = (((int64_t)hp + GN_T - 1) / GN_T) * (((int64_t)wp + GN_T - 1) / GN_T);
+  const int most = r <= 4 ? 1300 : r < 16 ? 700 : r <= 20 ? 1300 : r <= 32 ? 1000
+                   : r <= 128 ? 600 : 256;
+  return tiles <= most;
+}
+
 // The copies and interpolations below give a wave 256 columns, four per lane 64
 // apart (each access 256 contiguous bytes), and `walk` rows of them: what a
 // column or a pair of source rows determines is computed once per walk.  One
@@ -642,6 +837,19 @@ extern "C" int fsg_gaussian_nan(const fsg_window* src, int32_t pad, double sigma
   float* tw = (float*)((char*)workspace + need / 2);
   hipStream_t s = as_stream(stream);
   PadSrc S{src->data, src->ld, src->h, src->w, pad};
+  TimedScope ts("k_gauss_nan", s);
+  if (gauss_vector(hp, wp, G.r)) {
+    const dim3 grid((wp + GN_T - 1) / GN_T, (hp + GN_T - 1) / GN_T);
+    const size_t lds_r = sizeof(float) * (GN_T + 2 * G.r) * GN_T;
+    const size_t lds_c = sizeof(float) * GN_T * (GN_T + 2 * G.r + 1);
+    hipLaunchKernelGGL(k_gauss_tap_rows, grid, dim3(256), lds_r, s, S, G, tv, tw, (int64_t)wp,
+                       wconst);
+    FSG_CHECK_LAUNCH("k_gauss_tap_rows");
+    hipLaunchKernelGGL(k_gauss_tap_cols, grid, dim3(256), lds_c, s, tv, tw, (int64_t)wp, hp, wp,
+                       G, out, ldo, wconst, wdiv);
+    FSG_CHECK_LAUNCH("k_gauss_tap_cols");
+    return FSG_OK;
+  }
   const dim3 grid_r((wp + GN_T - 1) / GN_T, (hp + GN_L - 1) / GN_L);
   const dim3 grid_c((wp + GN_L - 1) / GN_L, (hp + GN_T - 1) / GN_T);
   const int ks_r = gn_ksteps(G.r, 4), ks_c = gn_ksteps(G.r, 16);
@@ -649,7 +857,6 @@ extern "C" int fsg_gaussian_nan(const fsg_window* src, int32_t pad, double sigma
   const size_t lds_r =
       sizeof(double) * ((4 * ks_r + 17) & ~1) + sizeof(float) * (112 + 4 * ks_r) * GN_T;
   const size_t lds_c = sizeof(double) * ((16 * ks_c + 17) & ~1) + sizeof(float) * GN_T * P;
-  TimedScope ts("k_gauss_nan", s);
   hipLaunchKernelGGL(k_gauss_nan_rows, grid_r, dim3(256), lds_r, s, S, G, ks_r, tv, tw,
                      (int64_t)wp);
   FSG_CHECK_LAUNCH("k_gauss_nan_rows");

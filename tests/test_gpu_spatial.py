@@ -277,11 +277,15 @@ def test_scheduler_stack_with_the_overview_and_uint8(cuda):
 
 
 @pytest.mark.parametrize("h,w,pad,sigma", [(1, 1, 0, 0.5), (64, 128, 0, 1.0), (129, 65, 3, 4.0),
-                                           (300, 257, 17, 10.25), (140, 513, 60, 40.0)])
+                                           (300, 257, 17, 10.25), (140, 513, 60, 40.0),
+                                           # extents of enough tiles for the band products
+                                           (1, 83300, 0, 0.5), (41665, 65, 0, 1.0),
+                                           (129, 28000, 3, 4.0), (6500, 300, 17, 10.25),
+                                           (140, 3300, 60, 40.0)])
 @pytest.mark.parametrize("special", ["none", "nan", "inf", "all_nan"])
 def test_gaussian_band_products_against_float64(cuda, h, w, pad, sigma, special):
-    """The band products at one-pixel, one-tile and ragged extents, for the fewest and the
-    most taps, against float64 sums: one float32 rounding per axis and of the quotient
+    """The vector sums (the first five extents) and the band products at one-pixel, one-tile
+    and ragged extents, for the fewest and the most taps, against float64 sums: one float32 rounding per axis and of the quotient
     (1.8e-7 relative of the largest weight sum).  An infinity reaches exactly the outputs
     whose taps cover it."""
     from fujishadergpu_amd import spatial
