@@ -407,10 +407,12 @@ __device__ __forceinline__ void box_t_block(const float* __restrict__ a,
   __syncthreads();
   // transposed write: output row = input column, output column = input row
   const int ncol = min(64, w - bx * 64);
-  for (int c0 = 0; c0 < ncol; c0 += 64 / BAND) {
-    const int cc = c0 + lane / BAND, k = lane % BAND;
-    const int y = y0 + k;
-    if (y < y1 && cc < ncol) {
+  const int k = BAND == 64 ? lane : lane % BAND, dc = BAND == 64 ? 0 : lane / BAND;
+  const int y = y0 + k;
+  if (y < y1) {
+    for (int c0 = 0; c0 < ncol; c0 += 64 / BAND) {
+      const int cc = c0 + dc;
+      if (cc >= ncol) break;
       const int64_t o = (int64_t)(bx * 64 + cc) * ldo + y;
       oa[o] = ta[k][cc];
       if (PASS == 0) ob[o] = tb[k][cc];
