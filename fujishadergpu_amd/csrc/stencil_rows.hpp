@@ -356,7 +356,7 @@ __device__ __forceinline__ void wave_lds_sync() {
 // in nan_fill's order, so the value is nan_fill's bits.  Bound: the float64
 // sums of the waves at a void's edge, which share a few SIMDs.  With every lane
 // summing its own four columns a 4096^2 curvature launch took 133 us at 1 % NoData
-// (80 without a void), hillshade or slope 108 (58); now 113 and 99.
+// (80 without a void); now 113.
 __device__ __forceinline__ void wave_fill4(const WinDev& W, int x, int cb, const float z[4],
                                            const bool want[4], const Gauss9& G, Fill4& L,
                                            float f[4]) {
@@ -456,10 +456,12 @@ __device__ __forceinline__ bool rows4_wave(const RowsTile4& S, int& c4, int& cb,
 // Hillshade and/or slope, four columns per lane.  Rows arrive one per
 // iteration from ra - 1 on; the first two iterations only fill (so the NaN
 // fill has one call site).
-// (The bound of six waves per SIMD keeps the fill from taking more registers
-// than the walk; five ran 3 % slower at 1 % NoData.)
+// (No bound on the waves per SIMD: held to the walk's registers the fill spilled and
+// had few loads in flight.  4096^2 hillshade without a void, with 1 % of discs and
+// with 30 % of single cells missing: 66, 110 and 364 us under a bound of six waves,
+// now 62, 108 and 317; slope 58, 102 and 360, now 56, 104 and 307.)
 template <bool NANAW>
-__global__ void __launch_bounds__(256, NANAW ? 6 : 1) k_shade_inner4(RowsTile4 S4, Gauss9 G) {
+__global__ void __launch_bounds__(256) k_shade_inner4(RowsTile4 S4, Gauss9 G) {
   constexpr int LEFT = SR4_LEFT_SHADE;
   int c4, cb, ra, rb;
   if (!rows4_wave<LEFT>(S4, c4, cb, ra, rb)) return;  // the whole wave
@@ -506,7 +508,7 @@ __global__ void __launch_bounds__(256, NANAW ? 6 : 1) k_shade_inner4(RowsTile4 S
                                     !isnan(right));
           any_want |= want[k];
         }
-        if (__ballot(any_want))  // the whole wave
+        if (__builtin_expect(__ballot(any_want) != 0, 0))  // the whole wave
           wave_fill4(S.W, r + 1, cb, zd, want, G, fill[threadIdx.x >> 6], fd);
         else
 #pragma unroll
