@@ -1055,22 +1055,9 @@ static int wave_rows(int rh, int n_strips, int capacity) {
   return std::max(16, (rh + segs - 1) / segs);
 }
 
-// Resident blocks of one k_usm_wave instance on the current device (CUs x
-// blocks per CU under its registers and LDS).
 template <int NR, int NS, int KR>
 static int wave_capacity() {
-  static const int cap = [] {
-    int dev = 0, cus = 0, nb = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-      cus = 256;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_usm_wave<NR, NS, KR>, 64, 0) !=
-            hipSuccess || nb <= 0) {
-      (void)hipGetLastError();
-      nb = 8;
-    }
-    return cus * nb;
-  }();
+  static const int cap = wave_resident(k_usm_wave<NR, NS, KR>);
   return cap;
 }
 
@@ -1582,18 +1569,7 @@ int fsg::usm_prep_jobs(const fsg_window* win, const fsg_topousm_params* p, void*
 // Resident blocks of one k_usm_wave_batch instance on the current device.
 template <int NS>
 static int wave_batch_capacity() {
-  static const int cap = [] {
-    int dev = 0, cus = 0, nb = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-      cus = 256;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_usm_wave_batch<3, NS, 1>, 64, 0) !=
-            hipSuccess || nb <= 0) {
-      (void)hipGetLastError();
-      nb = 8;
-    }
-    return cus * nb;
-  }();
+  static const int cap = wave_resident(k_usm_wave_batch<3, NS, 1>);
   return cap;
 }
 

@@ -408,6 +408,21 @@ __device__ __forceinline__ bool wave_tile(const WaveArgs& A, int tile, double* P
                                      Hc);
 }
 
+// Resident blocks of one wavefront kernel on the current device (CUs x blocks per
+// CU under its registers and LDS).
+template <class K>
+int wave_resident(K kernel) {
+  int dev = 0, cus = 0, nb = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    cus = 256;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, 64, 0) != hipSuccess || nb <= 0) {
+    (void)hipGetLastError();
+    nb = 8;
+  }
+  return cus * nb;
+}
+
 // The marked blocks of a k_usm_wave launch over the same arguments (usm_wave_nan.hip).
 int launch_wave_nan(const WaveArgs& A, int nr, int ns, hipStream_t s);
 

@@ -734,6 +734,9 @@ def test_wave_kernel_equals_the_workgroup_kernel(cuda, radii, weights, px, shape
     ([2, 8, 32], 10.0, (90, 300), (0, 0, 90, 300), False, "none", 0),
     ([2, 8, 32], 10.0, (9, 7), (0, 0, 9, 7), False, "pixel", 8),
     ([1], 10.0, (1, 1), (0, 0, 1, 1), False, "all", 0),
+    # windows past the line below which the marked blocks have 4 rows: 8 and 25 rows
+    ([2, 8, 32], 10.0, (2600, 3000), (0, 0, 2600, 3000), False, "scatter", 0),
+    ([2, 8, 32], 10.0, (2600, 3000), (7, 5, 2590, 2990), False, "disc", 200),
 ])
 def test_wave_kernel_on_nan_windows(cuda, radii, px, shape, reg, field, holes, variant):
     """A window with NaN: the wavefront kernel's plain blocks and the marked
