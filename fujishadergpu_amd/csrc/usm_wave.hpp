@@ -119,7 +119,9 @@ __device__ __forceinline__ int box_radius(const WaveArgs& A, int i) {
 // MODE WAVE_PLAIN: the plain means; WAVE_CHECK: with A.flags, returns true as
 // soon as the block has met a NaN or an infinity (its outputs are then
 // unfinished; an infinity makes NaN of every later running sum, so it too is
-// left to the shorter blocks); WAVE_NAN: the NaN-aware means.
+// left to the shorter blocks: it reaches the outputs of its strips from the row
+// above which no window meets it, R rows up, to at most 64 rows past the last that
+// does); WAVE_NAN: the NaN-aware means.
 enum { WAVE_PLAIN = 0, WAVE_CHECK = 1, WAVE_NAN = 2 };
 
 template <int NR, int NS, bool FAST, int KR, int MODE>

@@ -29,14 +29,16 @@ __global__ void __launch_bounds__(64) k_usm_wave_nan(WaveArgs A, int sub) {
 // radii 2, 8, 32 at 1 % of discs / 30 % of single cells missing, a call in us with 8
 // and with 4 rows: 512^2 89 / 58 and 78 / 48, 1700^2 104 / 78 and 96 / 94, 2400^2
 // (past the line) 120 / 124 and 109 / 144.  Else an eighth of a tile, 8 rows at
-// least.
-constexpr int WAVE_NAN_ROWS = 8, WAVE_NAN_FEW = 4;
+// least; at most 64, the workgroup kernels' block, since an infinity makes NaN of a
+// block's rows from where its sums meet it.
+constexpr int WAVE_NAN_ROWS = 8, WAVE_NAN_FEW = 4, WAVE_NAN_MOST = 64;
 
 template <int NR, int NS, int KR>
 static int launch(const WaveArgs& A, hipStream_t s) {
   static const int cap = wave_resident(k_usm_wave_nan<NR, NS, KR>);
   const bool few = (int64_t)A.n_strips * ((A.rh + WAVE_NAN_FEW - 1) / WAVE_NAN_FEW) <= 3 * cap;
-  const int sub = few ? WAVE_NAN_FEW : std::max(WAVE_NAN_ROWS, (A.SH + 7) / 8);
+  const int sub = few ? WAVE_NAN_FEW
+                      : std::min(WAVE_NAN_MOST, std::max(WAVE_NAN_ROWS, (A.SH + 7) / 8));
   TimedScope ts("k_usm_main", s);
   hipLaunchKernelGGL((k_usm_wave_nan<NR, NS, KR>), dim3(A.per_xcd * 8, (A.SH + sub - 1) / sub),
                      dim3(64), 0, s, A, sub);

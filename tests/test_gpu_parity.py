@@ -882,3 +882,35 @@ def test_valid_bbox_of_any_raster_on_the_gpu(cuda, kind):
     elif kind == "one_row_repeated":
         a, g = a[400:401].expand(900, 1700), g[400:401].expand(900, 1700)
     assert valid_bbox(g) == valid_bbox(a)
+
+
+@pytest.mark.parametrize("shape,variant", [((300, 700), 0), ((2600, 1500), 0), ((2600, 3000), 1024)])
+def test_infinity_in_a_nan_window_stays_near(cuda, shape, variant):
+    """An infinity makes NaN of running sums that meet it.  In a window with NaN it may
+    reach the outputs within R rows above it, 64 rows past the last window that holds it,
+    and one strip of 256 columns either side, whatever the blocks; every other output is
+    what a finite value in its place gives."""
+    from fujishadergpu_amd import ops
+    from fujishadergpu_amd.algorithms import OutSpec, TopoUSMFastAlgorithm
+    H, W = shape
+    R, yi, xi = 32, min(1000, H // 3), W // 2
+    dem = _dem(H, W, 23, relief=2000.0)
+    dem[H // 2:H // 2 + 5, 3:9] = float("nan")
+    p = dict(radii=[2, 8, R], weights=[1 / 3] * 3, pixel_size=10.0, global_stats=(19.5,),
+             _window_nan_free=False)
+    outs = []
+    try:
+        ops.set_topousm_variant(variant)
+        for v in (float("inf"), float(dem[yi, xi])):
+            g = dem.to(cuda)
+            g[yi, xi] = v
+            out = torch.empty((H, W), dtype=torch.float32, device=cuda)
+            TopoUSMFastAlgorithm().run_region(g, ops.region(0, 0, H, W), OutSpec(f32=out), p)
+            outs.append(out.cpu())
+    finally:
+        ops.set_topousm_variant(0)
+    far = torch.ones((H, W), dtype=torch.bool)
+    far[max(0, yi - R):yi + R + 65, max(0, xi - 256):xi + 257] = False
+    assert torch.equal(torch.nan_to_num(outs[0])[far], torch.nan_to_num(outs[1])[far])
+    assert torch.equal(torch.isnan(outs[0])[far], torch.isnan(dem)[far])
+    assert not torch.isfinite(outs[0][yi, xi])
