@@ -98,14 +98,15 @@ k_openness(WinDevR W, int r0, int c0, int rh, int rw, OpenTab T, OutDev out, Ray
 // the rays' reach around it, once, and samples that: address = the lane's +
 // one scalar per sample.  Samples outside the window are staged as the caller's
 // rule has them (NaN for openness, the edge for AO): no interior test.  What
-// bounds it now is VALU issue (16 directions of 50 pixels: about 36 operations
-// a pixel and direction).  8192^2, 16 directions of 50 pixels: 2714 us from
-// memory, now 1325; 8 of 64: 1534, 1037; 16 of 8: 2249, 935.
+// bounds it now is VALU issue: a difference, a product and an extreme per sample, and
+// an atanf per direction.  8192^2 from memory / staged, in us: 16 directions of 50
+// pixels 2737 / 1591, 8 of 64 1496 / 1231, 16 of 8 2248 / 1097.
 constexpr int RT_W = 128;             // tile columns: two per lane, 64 apart
 constexpr int RT_LDS = 160 * 1024;    // a CU's LDS
 constexpr int RT_LDS_HALF = 80 * 1024;
 constexpr int RT_PIECES = 5;          // 64-column pieces of a staged row
 constexpr int64_t RT_MIN_PX = 9 << 14;
+constexpr int64_t RT_MIN_PX_NEAR = (1 << 18) + 1;   // openness, a reach of 16 or less
 
 struct RayTile {
   RayGrid G;
@@ -116,18 +117,21 @@ struct RayTile {
 };
 
 // The tile of a region, or th = 0 where the reach leaves LDS no 16 rows (beyond
-// 68 pixels) or the region has fewer than 147456 pixels, where too few tiles
-// share the staging (256 x 512, 8 directions of 64: 13.6 us from memory, 15.5
-// staged; 100 x 1500: 16.2 and 15.4; 512^2: 19.8 and 16.0; AO the same line).  Two
-// tiles a CU where 48 rows or more fit half the LDS (one computes while the other
-// stages), else one of what fits; then the rows of the fewest full rounds of
-// tiles, spread evenly (regions of one round: down to 8 rows).
-inline RayTile ray_tile(int h, int w, int dy, int dx) {
+// 68 pixels) or the region has fewer than min_px pixels, where too few tiles share
+// the staging.  From memory / staged, in us: openness at 384^2, 16 directions of 50
+// pixels 25 / 17, 8 of 64 14.2 / 12.2, 8 of 24 11.9 / 10.1, but 16 of 16 13.6 / 15.1
+// and 8 of 8 8.1 / 9.3 (rays that stay in a few rows hit L1), at 512^2 14.0 / 15.0
+// and 8.5 / 9.3, at 576^2 24 / 17 and 13.4 / 11.3; at 300^2 8 of 64 11.4 / 12.1.  AO
+// with its smoothing at 384^2, 16 samples a ring of radius 10 30.5 / 25.6, 8 of 64
+// 23.8 / 24.2.  Two tiles a CU where 48 rows or more fit half the LDS (one computes
+// while the other stages), else one of what fits; then the rows of the fewest full
+// rounds of tiles, spread evenly (regions of one round: down to 8 rows).
+inline RayTile ray_tile(int h, int w, int dy, int dx, int64_t min_px = RT_MIN_PX) {
   RayTile R{};
   R.dy = dy;
   R.dx = dx;
   R.pitch = RT_W + 2 * dx;
-  if (R.pitch > 64 * RT_PIECES || w < 64 || (int64_t)h * w < RT_MIN_PX) return R;
+  if (R.pitch > 64 * RT_PIECES || w < 64 || (int64_t)h * w < min_px) return R;
   const int half = RT_LDS_HALF / 4 / R.pitch - 2 * dy, full = RT_LDS / 4 / R.pitch - 2 * dy;
   const int th = half >= 48 ? half : full, slots = half >= 48 ? 512 : 256;
   if (th < 16) return R;
@@ -703,7 +707,9 @@ extern "C" int fsg_openness(const fsg_window* win, const fsg_region* reg,
   if (reg->h == 0 || reg->w == 0) return FSG_OK;
   WinDevR W{win->data, win->ld, win->h, win->w};
   const RayTile R = T.n_dist >= 1 && T.n_dist <= OPEN_UNROLL
-                        ? ray_tile(reg->h, reg->w, T.dmax_y, T.dmax_x) : RayTile{};
+                        ? ray_tile(reg->h, reg->w, T.dmax_y, T.dmax_x,
+                                   std::max(T.dmax_y, T.dmax_x) <= 16 ? RT_MIN_PX_NEAR : RT_MIN_PX)
+                        : RayTile{};
   if (R.th)
     for (int e = 0; e < T.n_dirs * T.n_dist; e++) T.off[e] = lds_offset(T.off[e], R);
   const RayGrid G = R.th ? R.G : ray_grid(reg->h, reg->w, 4, 64);

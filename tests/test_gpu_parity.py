@@ -790,7 +790,9 @@ def test_wave_kernel_on_nan_windows(cuda, radii, px, shape, reg, field, holes, v
 
 @pytest.mark.parametrize("h,w,dist,n_dirs,typ", [
     (384, 384, 50, 16, "positive"), (2304, 64, 64, 8, "negative"), (1153, 128, 8, 33, "positive"),
-    (390, 389, 68, 3, "negative"), (385, 383, 69, 5, "positive"), (600, 257, 3, 1, "positive")])
+    (390, 389, 68, 3, "negative"), (385, 383, 69, 5, "positive"), (600, 257, 3, 1, "positive"),
+    # a reach of 16 or less: the last region that samples memory, the first staged ones
+    (512, 512, 16, 5, "positive"), (513, 513, 16, 5, "negative"), (1153, 256, 8, 33, "positive")])
 def test_openness_tiles_equal_the_pointwise_rays(cuda, h, w, dist, n_dirs, typ):
     """Regions large enough for the tiles staged in LDS (the reach at their limit and past
     it, one column panel and ragged ones, voids and the window's edges) against the
