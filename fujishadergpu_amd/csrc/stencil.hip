@@ -204,8 +204,11 @@ static RowsTile rows_tile(const StencilTile& S, const fsg_region* reg, const Rec
 }
 
 // The general kernels (every position, numpy's edge formulas included) over
-// up to RS_MAX rectangles of the region, one launch: hillshade/slope (one
-// lane per pixel with NaN, a row walk without) or curvature (tiled block).
+// up to RS_MAX rectangles of the region, one launch: the tiled block (curvature,
+// and hillshade/slope over a whole NaN-aware region: 256^2 to 1000^2 without a void
+// as long as one lane per pixel, with 1 % of discs 16 to 20 us against 27 to 42), or
+// for hillshade/slope one lane per pixel (the border strips of a NaN-aware window) or
+// a row walk (without NaN).
 static void launch_general(const StencilTile& S, const Rect* q, int n, bool tiled,
                            hipStream_t s) {
   const int bh = tiled ? ST_TH : (S.nanaw ? 4 : 4 * SHADE_R);
@@ -230,9 +233,14 @@ static void launch_general(const StencilTile& S, const Rect* q, int n, bool tile
 // hide its loads (2048^2 windows ran faster as one general launch).
 constexpr int64_t SPLIT_MIN_DEFAULT = int64_t(1) << 23;
 static std::atomic<int64_t> g_split_min{SPLIT_MIN_DEFAULT};
-// NaN-aware windows take the row kernels from 2^20 interior pixels (or the
-// process-wide setting, when smaller).
-constexpr int64_t SPLIT_MIN_NANAW = int64_t(1) << 20;
+// NaN-aware windows take the row kernels from 3 * 2^20 interior pixels (or the
+// process-wide setting, when smaller): the tiled block shares its fills, so small
+// launches wait for a void's edge less than row walks do.  A call in us, rows /
+// tiled, without a void and with 1 % of discs: 1100^2 hillshade 24 / 15 and 58 / 21,
+// slope 22 / 14 and 57 / 20, curvature 35 / 20 and 59 / 26; 1500^2 26 / 22 and 64 /
+// 29, 24 / 21 and 62 / 28, 36 / 31 and 63 / 37; 2048^2 31 / 34 and 66 / 41, 28 / 32
+// and 64 / 40, 40 / 48 and 64 / 55: without a void the rows win from about 1770^2 on.
+constexpr int64_t SPLIT_MIN_NANAW = int64_t(3) << 20;
 
 // Constant-step hillshade/slope or curvature: the row-walking kernel over
 // the interior, then ONE general launch over the border strips (and the

@@ -192,7 +192,7 @@ def _stencils_wide_windows(cuda, nan_discs, off, ld):
 
 @pytest.mark.parametrize("h,w,holes", [
     (203, 517, "discs"), (64, 300, "scatter"), (17, 1040, "edges"), (70, 259, "lines"),
-    (150, 390, "islands"),
+    (150, 390, "islands"), (1030, 1100, "scatter"), (1500, 1531, "lines"),
 ])
 def test_nan_fills_of_row_and_tile_kernels_agree(cuda, h, w, holes):
     """The fill shared by a wave (row kernels) and by a block (tiled kernel),
