@@ -916,3 +916,26 @@ def test_infinity_in_a_nan_window_stays_near(cuda, shape, variant):
     assert torch.equal(torch.nan_to_num(outs[0])[far], torch.nan_to_num(outs[1])[far])
     assert torch.equal(torch.isnan(outs[0])[far], torch.isnan(dem)[far])
     assert not torch.isfinite(outs[0][yi, xi])
+
+
+@pytest.mark.parametrize("h,w,samples,radius", [(500, 420, 16, 10.0), (480, 389, 7, 33.0),
+                                                (600, 260, 61, 3.0), (390, 400, 8, 64.0)])
+def test_ambient_occlusion_tiles_equal_the_direct_kernel(cuda, h, w, samples, radius):
+    """A region large enough for the tiles staged in LDS against the same pixels as bands
+    that sample memory: the same bits, at voids, infinities and the window's edges."""
+    from fujishadergpu_amd import ops, synth
+    from fujishadergpu_amd.algorithms import ao_samples
+    dem = synth.fbm(h + 9, w + 6, 0.7, 400.0, seed=8, device="cuda")
+    synth.apply_discs(dem, [(h // 2, w // 3, 21), (30, w - 5, 20), (0, 0, 9)], float("nan"))
+    dem[h // 4, w // 4], dem[h // 4 + 2, w // 4 + 1] = float("inf"), float("-inf")
+    table = ao_samples(samples, radius, 2.0)
+    pad = max(1, int(round(radius)))
+
+    def run(r0, rows):
+        out = torch.empty((rows, w), device=cuda)
+        ops.ambient_occlusion(dem, ops.region(r0, 3, rows, w), table=table, intensity=1.0,
+                              pad_d=pad, out=ops.output(out))
+        return out
+    got = run(0, h)
+    want = torch.cat([run(r, min(90, h - r)) for r in range(0, h, 90)])
+    assert torch.equal(got.view(torch.int32), want.view(torch.int32))
