@@ -17,7 +17,7 @@ FSG_OK, FSG_E_INVALID, FSG_E_HIP, FSG_E_UNSUPPORTED, FSG_E_WORKSPACE = 0, 1, 2, 
 OUT_F32, OUT_I16, OUT_U8 = 0, 1, 2
 POST_NONE, POST_DIV, POST_STRETCH = 0, 1, 2
 MAX_RADII = 16
-ABI_VERSION = 20  # FSG_ABI_VERSION of include/fsg.h
+ABI_VERSION = 21  # FSG_ABI_VERSION of include/fsg.h
 
 
 class NativeLibraryError(RuntimeError):
@@ -324,6 +324,9 @@ def lib():
             L = C.CDLL(LIB_PATH)
         except OSError as exc:
             raise NativeLibraryError(f"cannot load {LIB_PATH}: {exc}") from exc
+        # the version before the symbols: an older library lacks some
+        if not hasattr(L, "fsg_abi_version") or L.fsg_abi_version() != ABI_VERSION:
+            raise NativeLibraryError(f"{LIB_PATH}: ABI version mismatch (need {ABI_VERSION})")
         for name, (res, args) in _SIGS.items():
             try:
                 fn = getattr(L, name)
@@ -331,8 +334,6 @@ def lib():
                 raise NativeLibraryError(f"{LIB_PATH} lacks symbol {name}") from exc
             fn.restype = res
             fn.argtypes = args
-        if L.fsg_abi_version() != ABI_VERSION:
-            raise NativeLibraryError("libfsg.so ABI version mismatch")
         _lib = L
         return _lib
 

@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define FSG_ABI_VERSION 20
+#define FSG_ABI_VERSION 21
 
 enum {
   FSG_OK = 0,

@@ -23,7 +23,7 @@ def test_binding_table_covers_header():
 
 def test_loader_validates_abi_and_symbols():
     L = N.lib()
-    assert L.fsg_abi_version() == N.ABI_VERSION == 20
+    assert L.fsg_abi_version() == N.ABI_VERSION == 21
     assert L.fsg_launch_count() >= 0
 
 
@@ -89,3 +89,21 @@ def test_ctypes_layout_matches_the_c_header(tmp_path):
         assert int(got[f"{name} size"]) == ctypes.sizeof(st), name
         for f in st._fields_:
             assert int(got[f"{name}.{f[0]}"]) == getattr(st, f[0]).offset, f"{name}.{f[0]}"
+
+
+def test_older_library_is_refused_by_its_version(tmp_path, monkeypatch):
+    """A library of the version before, which lacks the newer entry points, is refused by
+    its version and not by the first symbol that it lacks."""
+    import importlib
+    import subprocess
+    src, so = tmp_path / "old.c", tmp_path / "old.so"
+    src.write_text("int fsg_abi_version(void) { return 20; }\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(src)], check=True)
+    monkeypatch.setenv("FSG_LIBRARY", str(so))
+    mod = importlib.reload(N)
+    try:
+        with pytest.raises(mod.NativeLibraryError, match="ABI version"):
+            mod.lib()
+    finally:
+        monkeypatch.delenv("FSG_LIBRARY")
+        importlib.reload(N)
