@@ -34,7 +34,7 @@ from . import _native as N
 from . import ops
 from .algorithms import (CurvatureAlgorithm, HillshadeAlgorithm, OpennessAlgorithm, OutSpec,
                          SlopeAlgorithm, TopoUSMFastAlgorithm, _post_from_stats, curvature_steps,
-                         gradient_steps, openness_table, x_steps_rows)
+                         gradient_steps, openness_samples, x_steps_rows)
 from .params import DEFAULT_ALTITUDE, DEFAULT_AZIMUTH
 
 
@@ -135,9 +135,9 @@ def _tile_struct(job: TileJob, keep: list) -> N.fsg_batch_tile:
     t.topousm2 = _empty_out()
     if job.openness is not None:
         p = pp.get("openness", job.params)
-        table = openness_table(p.get("num_directions", 16), p.get("max_distance", 50),
-                               p.get("pixel_size", 1.0), p.get("pixel_scale_x"),
-                               p.get("pixel_scale_y"))
+        table = openness_samples(p.get("num_directions", 16), p.get("max_distance", 50),
+                                 p.get("pixel_size", 1.0), p.get("pixel_scale_x"),
+                                 p.get("pixel_scale_y"))
         prm, arr = ops.openness_params(table, p.get("openness_type", "positive"), False)
         keep.append(arr)
         t.open = prm

@@ -626,7 +626,9 @@ k_ao_smooth(AoSmooth A, Gauss9 G, OutDev out) {
   const PostK pp = load_post(out);
   const bool writes = lane >= 1 && lane <= 62 && c < A.rw;
   const int n = min(4, A.rw - c);
-  double x[4][17];   // per column: rows i - 4 .. i + 12 of the batch
+  // the rows come in batches of AO_SB: their loads are issued together
+  constexpr int AO_SB = 4;
+  double x[4][8 + AO_SB];   // per column: rows y - 4 .. y + 3 + AO_SB around the batch at y
 #pragma unroll
   for (int k = 0; k < 8; k++) {
     float v[4];
@@ -634,8 +636,6 @@ k_ao_smooth(AoSmooth A, Gauss9 G, OutDev out) {
 #pragma unroll
     for (int m = 0; m < 4; m++) x[m][k] = (double)v[m];
   }
-  // the rows come in batches of AO_SB: their loads are issued together
-  constexpr int AO_SB = 4;
   for (int yb = 0; yb < rows; yb += AO_SB) {
     float f[AO_SB][4], zz[AO_SB][4];
 #pragma unroll

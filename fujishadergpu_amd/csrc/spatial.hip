@@ -46,8 +46,8 @@ struct PadSrc {
 };
 
 // The NaN-aware Gaussian runs as two LDS-tiled passes over output tiles of 128 along
-// the filter axis and 64 across it, each a product with a band matrix in float64 on the matrix cores
-// (v_mfma_f64_16x16x4_f64: lane l holds A[l % 16][l / 16], B[l / 16][l % 16] and,
+// the filter axis and 64 across it, each a product with a band matrix in float64 on
+// the matrix cores (v_mfma_f64_16x16x4_f64: lane l holds A[l % 16][l / 16], B[l / 16][l % 16] and,
 // in entry e, D[l / 16 + 4 e][l % 16]): T[y][k] = g[|k - y - r|] over the 16 + 2 r
 // samples that 16 outputs reach, zero outside the band, so the LDS span past a
 // window of taps must be finite.  Sums stay float64; only their order is the

@@ -56,24 +56,6 @@ __device__ __forceinline__ void nan_fill_col(const WinDev& W, int r, int cc, con
   fw = (float)sw;
 }
 
-// The axis-0 pass from the column's nine values, rows r - 4 .. r + 4 (clamped).
-__device__ __forceinline__ void nan_fill_sum(const float v[9], const Gauss9& G, float& fv,
-                                             float& fw) {
-  const bool v0 = !isnan(v[4]);
-  double sv = (v0 ? (double)v[4] : 0.0) * G.g[0];
-  double sw = (v0 ? 1.0 : 0.0) * G.g[0];
-#pragma unroll
-  for (int d = 4; d >= 1; d--) {
-    const float a = v[4 - d], b = v[4 + d];
-    const double fa = isnan(a) ? 0.0 : (double)a, fb = isnan(b) ? 0.0 : (double)b;
-    const double wa = isnan(a) ? 0.0 : 1.0, wb = isnan(b) ? 0.0 : 1.0;
-    sv += (fa + fb) * G.g[d];
-    sw += (wa + wb) * G.g[d];
-  }
-  fv = (float)sv;
-  fw = (float)sw;
-}
-
 // The axis-1 pass at ce from the column sums around it.
 __device__ __forceinline__ float nan_fill_row(const float2* ce, const Gauss9& G) {
   double sv = (double)ce->x * G.g[0];

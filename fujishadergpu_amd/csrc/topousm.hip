@@ -1212,7 +1212,7 @@ struct CoarsePlan {
   size_t grid_off[FSG_MAX_RADII];   // per distinct ds: decimated grid
   size_t mean_off[FSG_MAX_RADII];   // per radius: coarse mean grid
   size_t flag_off;
-  size_t tmp_off[4];
+  size_t tmp_off[3];
   size_t total = 0;
   int max_cells = 0;
   int max_vrad = 0;
@@ -1251,7 +1251,7 @@ static CoarsePlan plan_coarse(const fsg_window* win, const fsg_topousm_params* p
   }
   P.flag_off = off;
   off += align256(sizeof(int) * FSG_MAX_RADII);
-  for (int k = 0; k < 4; k++) {
+  for (int k = 0; k < 3; k++) {
     P.tmp_off[k] = off;
     off += align256(sizeof(float) * (size_t)P.max_cells);
   }
@@ -1423,8 +1423,8 @@ int fsg::usm_prepare(const fsg_window* win, const fsg_region* reg, const fsg_top
 
   // coarse grids for ds > 1 radii
   int* flags = (int*)(ws + P.flag_off);
-  float* tmp[4];
-  for (int k = 0; k < 4; k++) tmp[k] = (float*)(ws + P.tmp_off[k]);
+  float* tmp[3];
+  for (int k = 0; k < 3; k++) tmp[k] = (float*)(ws + P.tmp_off[k]);
   for (int j = 0; j < P.n_ds && launch_prep; j++) {
     rc = decimate(win, P.ds_val[j], (float*)(ws + P.grid_off[j]), P.hc[j], P.wc[j], flags + j,
                   tmp[0], tmp[1], tmp[2], p->nan_hint == 0, s);
@@ -1701,7 +1701,7 @@ int fsg::launch_box_batch(int pass, const BoxJob* jobs, const int* pre, int n_jo
 extern "C" size_t fsg_downsample_workspace_size(int32_t h, int32_t w, int32_t factor) {
   if (h <= 0 || w <= 0 || factor < 1) return 0;
   const size_t cells = (size_t)((h + factor - 1) / factor) * (size_t)((w + factor - 1) / factor);
-  return 4 * align256(sizeof(float) * cells) + align256(sizeof(int) * 4);
+  return 3 * align256(sizeof(float) * cells) + align256(sizeof(int) * 4);
 }
 
 extern "C" int fsg_downsample_nan_aware(const fsg_window* src, int32_t factor, float* out,
@@ -1720,9 +1720,9 @@ extern "C" int fsg_downsample_nan_aware(const fsg_window* src, int32_t factor, f
     return fail(FSG_E_WORKSPACE, "fsg_downsample_nan_aware: workspace too small");
   char* ws = (char*)workspace;
   const size_t g = align256(sizeof(float) * (size_t)hc * wc);
-  float* t[4];
-  for (int k = 0; k < 4; k++) t[k] = (float*)(ws + k * g);
-  int* flag = (int*)(ws + 4 * g);
+  float* t[3];
+  for (int k = 0; k < 3; k++) t[k] = (float*)(ws + k * g);
+  int* flag = (int*)(ws + 3 * g);
   return decimate(src, factor, out, hc, wc, flag, t[0], t[1], t[2], false,
                   as_stream(stream));
 }
@@ -1805,8 +1805,8 @@ extern "C" int fsg_topousm_noalloc(const fsg_window* win, const fsg_region* reg,
 extern "C" size_t fsg_topousm_coarse_means_workspace_size(const fsg_window* win, int32_t ds) {
   if (!win || win->h <= 0 || win->w <= 0 || ds < 1) return 0;
   const size_t cells = (size_t)((win->h + ds - 1) / ds) * (size_t)((win->w + ds - 1) / ds);
-  // decimated grid, flag, four void-fill temporaries (two reused by the box passes)
-  return 5 * align256(sizeof(float) * cells) + align256(sizeof(int) * 4);
+  // decimated grid, flag, three void-fill temporaries (two reused by the box passes)
+  return 4 * align256(sizeof(float) * cells) + align256(sizeof(int) * 4);
 }
 
 extern "C" int fsg_topousm_coarse_means(const fsg_window* win, int32_t ds, int32_t n_radii,
@@ -1828,9 +1828,9 @@ extern "C" int fsg_topousm_coarse_means(const fsg_window* win, int32_t ds, int32
   char* ws = (char*)workspace;
   const size_t g = align256(sizeof(float) * (size_t)hc * wc);
   float* grid = (float*)ws;
-  float* tmp[4];
-  for (int k = 0; k < 4; k++) tmp[k] = (float*)(ws + (1 + k) * g);
-  int* flag = (int*)(ws + 5 * g);
+  float* tmp[3];
+  for (int k = 0; k < 3; k++) tmp[k] = (float*)(ws + (1 + k) * g);
+  int* flag = (int*)(ws + 4 * g);
   hipStream_t s = as_stream(stream);
   int64_t ldg = wc;
   if (ds == 1) {  // the window is already the grid

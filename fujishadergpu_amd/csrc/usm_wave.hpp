@@ -102,12 +102,12 @@ __device__ __forceinline__ double bits_f64(int lo, int hi) {
   return __builtin_bit_cast(double, ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
 }
 
-// `rows` rows of a strip (at most SW columns) of the region.  P: this wave's LDS prefix buffer (4 *
-// WAVE_PB doubles, one radius at a time).  Hc: its LDS copy of the float64
-// coarse-row values of each source, [NS][2][WAVE_NC] (lane t uses columns
-// 4t .. 4t + 3 only).  FAST: every row and column the block reads lies inside
-// the window (no reflection); a lane's four columns are one 16-byte load,
-// dword-aligned (gfx9 and later take it as one access at any column).
+// `rows` rows of a strip (at most SW columns) of the region.  P: this wave's LDS
+// prefix buffer (4 * WAVE_PB doubles, one radius at a time).  Hc: its LDS copy of the
+// float64 coarse-row values of each source, [NS][2][WAVE_NC] (lane t uses columns
+// 4t .. 4t + 3 only).  FAST: every row and column the block reads lies inside the
+// window (no reflection); a lane's four columns are one 16-byte load, dword-aligned
+// (gfx9 and later take it as one access at any column).
 // KR = 1: the box radii are {2, 8, 32} (every prefix-entry offset an
 // immediate); KR = 0: the radii of A.
 template <int KR>

@@ -599,7 +599,8 @@ int fsg_combine_fields(const float* const* fields, int32_t n, int64_t ld, const 
  * fsg_cnn_conv3x3_wgrad accumulates dw [32][cin][9] and db [32] (f32; zero
  * them first) from the layer input x and the pre-activation gradient dz
  * [..][32] bf16; the _ws form sums its workgroups' partials through a
- * workspace of fsg_cnn_wgrad_workspace_size bytes instead of by atomics.  fsg_cnn_pack writes the forward and (wt != NULL) backward
+ * workspace of fsg_cnn_wgrad_workspace_size bytes instead of by atomics.
+ * fsg_cnn_pack writes the forward and (wt != NULL) backward
  * bf16 layouts of float32 weights w [cout][cin][3][3].  fsg_cnn_adam is one
  * bias-corrected Adam step on float32 parameters (step counts from 1).
  */
