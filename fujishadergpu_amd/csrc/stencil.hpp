@@ -390,13 +390,20 @@ __device__ __forceinline__ void stencil_tile_block_v(const StencilTile& S, int b
 #pragma unroll
         for (int j = 0; j < NCW; j++) {
           const int rr = (t >> 6) + 4 * i, cc = (t & 63) + 64 * j;
-          if (rr < nr && cc < nc) {
-            hole |= isnan(v[i][j]);
-            valid |= !isnan(v[i][j]) & (tr0 + rr >= rl) & (tr0 + rr < rl + rows) &
-                     (tc0 + cc >= cl) & (tc0 + cc < cl + cols);
-          }
+          if (rr < nr && cc < nc) hole |= isnan(v[i][j]);
         }
-      if (__syncthreads_or(hole) && __syncthreads_or(valid)) {
+      const bool any_hole = __syncthreads_or(hole);
+      if (any_hole) {
+#pragma unroll
+        for (int i = 0; i < NRW; i++)
+#pragma unroll
+          for (int j = 0; j < NCW; j++) {
+            const int rr = (t >> 6) + 4 * i, cc = (t & 63) + 64 * j;
+            valid |= (rr < nr) & (cc < nc) & !isnan(v[i][j]) & (tr0 + rr >= rl) &
+                     (tr0 + rr < rl + rows) & (tc0 + cc >= cl) & (tc0 + cc < cl + cols);
+          }
+      }
+      if (any_hole && __syncthreads_or(valid)) {
         constexpr int FW = ST_TW + 2 * ST_HALO + 8;             // column sums of a row
         constexpr int NAN_ROWS = (2 * ST_PH * ST_PW) / (2 * FW);  // rows that fit
         static_assert(ST_ROWS * ST_LT % 2 == 0, "the sums are float2 from Pt on");
